@@ -10,6 +10,7 @@ const SOURCES: &[&str] = &[
         "rv_decode.hip",
         "rv_prefill.hip",
         "rv_quant.hip",
+        "rv_batched.hip",
         "rv_gemv_abi.cpp",
         "rv_block_abi.cpp",
         "rv_router.hip",

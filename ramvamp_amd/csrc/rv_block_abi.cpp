@@ -150,8 +150,7 @@ int32_t rv_attn_block_prefill(rv_kv* kv, size_t layer, float* residual_rows, siz
   if (hidden == 0) return fail(err, RV_PRIM_EMPTY, 0, 0, "rmsnorm");
   const size_t kv_dim = kv->kv_dim, n = n_rows;
   char* p = (char*)scratch;
-  float* normed = (float*)p;
-  p += align256(n * hidden * 4);
+  p += align256(n * hidden * 4);  // (held the normed rows; the quantizer norms them now)
   float* q = (float*)p;
   p += align256(n * q_dim * 4);
   float* k = (float*)p;
@@ -160,7 +159,7 @@ int32_t rv_attn_block_prefill(rv_kv* kv, size_t layer, float* residual_rows, siz
   p += align256(n * kv_dim * 4);
   float* attn = (float*)p;
   p += align256(n * q_dim * 4);
-  rv::InProj in{normed, nullptr, 0.f, hidden, w->q_format, w->wq, 0, q, q_dim, w->wk, 0, k, kv_dim,
+  rv::InProj in{residual_rows, w->attn_norm, eps, hidden, w->q_format, w->wq, 0, q, q_dim, w->wk, 0, k, kv_dim,
                 w->v_format, w->wv, 0, v, p};
   int32_t rc;
   if ((rc = rv::in_proj_rows_check(in, n, w->wq_len, w->wk_len, w->wv_len, err))) return rc;
@@ -187,8 +186,7 @@ int32_t rv_attn_block_prefill(rv_kv* kv, size_t layer, float* residual_rows, siz
   if (hipGetDevice(&prev) != hipSuccess) prev = -1;
   if (prev != kv->device) (void)hipSetDevice(kv->device);
   const hipStream_t s = kv->stream;
-  rv::HipStatus st = rv::launch_rmsnorm_rows(residual_rows, w->attn_norm, eps, n, hidden, normed, s);
-  if (st.e == hipSuccess) st = rv::in_proj_rows_launch(in, n, s);
+  rv::HipStatus st = rv::in_proj_rows_launch(in, n, s);
   if (st.e != hipSuccess) rc = fail(err, RV_ERR_HIP, (uint64_t)st.e, 0, st.what);
   if (!rc)
     rc = rv_prefill_chunk(kv, layer, q, k, v, n, q_dim, w->q_norm, w->q_norm_len, w->k_norm, w->k_norm_len, eps, theta, start, scale, attn,

@@ -53,6 +53,15 @@ int32_t finish(hipStream_t s, uint32_t flags, const rv::HipStatus& st, rv_error*
 
 bool k_quant(uint32_t f) { return f == RV_QF_Q4_K || f == RV_QF_Q5_K || f == RV_QF_Q6_K; }
 
+// One matrix over activation rows in the public block layout, stored
+// out[i * n_acts + a].
+rv::BatchedArgs batched_args(uint32_t fmt, const uint8_t* w, size_t row_bytes, size_t in_dim, const void* acts,
+                             size_t n_acts, size_t row_lo, size_t n_rows, float* out) {
+  return rv::BatchedArgs{1,
+                         {{fmt, w, row_bytes, (long)row_lo, (int)n_rows, out, (long)n_acts, 0, 0}},
+                         acts, acts, (int)n_acts, (int)in_dim, 0, 0, 0};
+}
+
 // quantize.rs check_len (:11-26).
 int32_t check_quantize(uint32_t format, size_t floats, size_t out_blocks, rv_error* err) {
   const size_t width = format == RV_QF_Q8_0 ? 32 : 256;
@@ -212,8 +221,9 @@ int32_t rv_gemv_q8_k_batched(uint32_t format, const uint8_t* weight, size_t weig
   if ((rc = check_ptrs(err, {{weight, "weight"}, {acts, "acts"}, {out, "out"}}))) return rc;
   const hipStream_t s = (hipStream_t)stream;
   return finish(s, flags,
-                rv::launch_gemv_batched(format, weight, row_bytes, in_dim, acts, n_acts, row_lo, row_hi - row_lo, out,
-                                        n_acts, false, s),
+                rv::launch_batched(batched_args(format, weight, row_bytes, in_dim, acts, n_acts, row_lo,
+                                                row_hi - row_lo, out),
+                                   false, s),
                 err);
 }
 
@@ -228,8 +238,9 @@ int32_t rv_gemv_q8_0_batched(const uint8_t* weight, size_t weight_len, size_t in
   if ((rc = check_ptrs(err, {{weight, "weight"}, {acts, "acts"}, {out, "out"}}))) return rc;
   const hipStream_t s = (hipStream_t)stream;
   return finish(s, flags,
-                rv::launch_gemv_batched(RV_QF_Q8_0, weight, row_bytes, in_dim, acts, n_acts, row_lo,
-                                        row_hi - row_lo, out, n_acts, false, s),
+                rv::launch_batched(batched_args(RV_QF_Q8_0, weight, row_bytes, in_dim, acts, n_acts, row_lo,
+                                                row_hi - row_lo, out),
+                                   false, s),
                 err);
 }
 
@@ -467,27 +478,27 @@ int32_t out_proj_rows_check(OutProj& p, size_t n, size_t wo_len, rv_error* err) 
 }
 
 HipStatus in_proj_rows_launch(const InProj& p, size_t n, hipStream_t s) {
-  auto* acts_k = reinterpret_cast<rv_block_q8_k*>(p.scratch);
-  auto* acts_0 =
-      reinterpret_cast<rv_block_q8_0*>((char*)p.scratch + align16(n * (p.hidden / 256) * sizeof(rv_block_q8_k)));
-  // A row of hidden values is a whole number of blocks of both forms, so the
-  // rows quantized one after another are one quantization of their concatenation.
-  HipStatus st = launch_quantize_both(p.x, acts_k, acts_0, n * (p.hidden / 256), s);
-  if (st.e == hipSuccess)
-    st = launch_gemv_batched(p.q_format, p.wq, p.rb_q, p.hidden, acts_k, n, 0, p.q_dim, p.q, p.q_dim, true, s);
-  if (st.e == hipSuccess)
-    st = launch_gemv_batched(RV_QF_Q8_0, p.wk, p.rb_k, p.hidden, acts_0, n, 0, p.kv_dim, p.k, p.kv_dim, true, s);
-  if (st.e == hipSuccess)
-    st = launch_gemv_batched(p.v_format, p.wv, p.rb_v, p.hidden, acts_k, n, 0, p.kv_dim, p.v, p.kv_dim, true, s);
-  return st;
+  void* acts_k = p.scratch;
+  void* acts_0 = (char*)p.scratch + align16(n * (p.hidden / 256) * sizeof(rv_block_q8_k));
+  HipStatus st = launch_quantize_rows(p.x, n, p.hidden, p.norm_w, p.eps, acts_k, acts_0, s);
+  if (st.e != hipSuccess) return st;
+  // k first: its per-block float chain is eight times as long as the
+  // k-quants', so its workgroups start before q's.
+  BatchedArgs a{3,
+                {{RV_QF_Q8_0, p.wk, p.rb_k, 0, (int)p.kv_dim, p.k, (long)p.kv_dim, 0, 0},
+                 {p.v_format, p.wv, p.rb_v, 0, (int)p.kv_dim, p.v, (long)p.kv_dim, 0, 0},
+                 {p.q_format, p.wq, p.rb_q, 0, (int)p.q_dim, p.q, (long)p.q_dim, 0, 0}},
+                acts_k, acts_0, (int)n, (int)p.hidden, 1, 0, 0};
+  return launch_batched(a, true, s);
 }
 
 HipStatus out_proj_rows_launch(const OutProj& p, size_t n, hipStream_t s) {
-  auto* acts = reinterpret_cast<rv_block_q8_k*>(p.scratch);
-  HipStatus st = launch_quantize_q8_k(p.x, acts, n * (p.q_dim / 256), s);
-  if (st.e == hipSuccess)
-    st = launch_gemv_batched(p.o_format, p.wo, p.rb, p.q_dim, acts, n, 0, p.hidden, p.o, p.hidden, true, s, true);
-  return st;
+  HipStatus st = launch_quantize_rows(p.x, n, p.q_dim, nullptr, 0.f, p.scratch, nullptr, s);
+  if (st.e != hipSuccess) return st;
+  BatchedArgs a{1,
+                {{p.o_format, p.wo, p.rb, 0, (int)p.hidden, p.o, (long)p.hidden, 0, 0}},
+                p.scratch, nullptr, (int)n, (int)p.q_dim, 1, 1, 0};
+  return launch_batched(a, true, s);
 }
 
 }  // namespace rv

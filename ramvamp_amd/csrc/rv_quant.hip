@@ -226,56 +226,53 @@ __device__ __forceinline__ float q80_row(const uint8_t* __restrict__ row, int nb
 }
 
 // quantize_row_q8_k (quantize.rs:71-106) of one block by one wave, lane l
-// holding values 4l .. 4l+3: the first value of largest magnitude (per lane
-// in order, then across lanes by magnitude and lowest index; magnitudes of
-// 0 and NaN never win, as `av > amax` from amax = 0 never takes them), RNE
-// rounding, the clamp, bsums, and the scalar code's f32 divisions.
+// holding values 4l .. 4l+3: the first value of largest magnitude (the
+// maximum over the wave, then the lowest lane that holds it and that lane's
+// first such value; NaN never wins, as `av > amax` never takes it), RNE
+// rounding, the clamp, the sums of 16 values and the scalar code's f32
+// divisions. A block whose maximum is 0 is all zeros.
+struct Q8KLane {
+  uint32_t q;  // the lane's four quants
+  int sum16;   // the sum over its aligned group of four lanes (16 values)
+  float d;
+};
+__device__ __forceinline__ Q8KLane quantize_lane_q8_k(const float (&v)[4]) {
+  float amax = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(v[e]));
+  amax = swap_max<32>(swap_max<16>(group_max<16>(amax)));
+  Q8KLane r{0u, 0, 0.f};
+  if (amax == 0.f) return r;  // wave-uniform
+  float first = 0.f;
+  bool any = false;
+#pragma unroll
+  for (int e = 3; e >= 0; --e)
+    if (fabsf(v[e]) == amax) {
+      first = v[e];
+      any = true;
+    }
+  const float mx = lane_f(first, __builtin_ctzll(__ballot(any)));
+  const float iscale = -127.f / mx;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int n = min(max((int)__builtin_rintf(iscale * v[e]), -128), 127);
+    r.q |= (uint32_t)(n & 0xFF) << (8 * e);
+    r.sum16 += n;
+  }
+  r.sum16 += __builtin_amdgcn_update_dpp(0, r.sum16, DPP_QUAD_XOR1, 0xF, 0xF, false);
+  r.sum16 += __builtin_amdgcn_update_dpp(0, r.sum16, DPP_QUAD_XOR2, 0xF, 0xF, false);
+  r.d = 1.f / iscale;
+  return r;
+}
+
 __device__ __forceinline__ void quantize_block_q8_k(const float* __restrict__ xs, rv_block_q8_k* blk, int lane) {
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = xs[4 * lane + e];
-  float amax = 0.f, mx = 0.f;
-  int idx = 1 << 30;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float av = fabsf(v[e]);
-    if (av > amax) {
-      amax = av;
-      mx = v[e];
-      idx = 4 * lane + e;
-    }
-  }
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const float a2 = __shfl_xor(amax, off, 64), m2 = __shfl_xor(mx, off, 64);
-    const int i2 = __shfl_xor(idx, off, 64);
-    if (a2 > amax || (a2 == amax && i2 < idx)) {
-      amax = a2;
-      mx = m2;
-      idx = i2;
-    }
-  }
-  if (amax == 0.f) {  // wave-uniform
-    *reinterpret_cast<uint32_t*>(blk->qs + 4 * lane) = 0u;
-    if (lane < 16) blk->bsums[lane] = 0;
-    if (lane == 0) blk->d = 0.f;
-    return;
-  }
-  const float iscale = -127.f / mx;
-  uint32_t packed = 0;
-  int gsum = 0;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int n = min(max((int)__builtin_rintf(iscale * v[e]), -128), 127);
-    packed |= (uint32_t)(n & 0xFF) << (8 * e);
-    gsum += n;
-  }
-  *reinterpret_cast<uint32_t*>(blk->qs + 4 * lane) = packed;
-  // bsums[g]: the 16 values of lanes 4g .. 4g+3.
-  gsum += __shfl_xor(gsum, 1, 64);
-  gsum += __shfl_xor(gsum, 2, 64);
-  if ((lane & 3) == 0) blk->bsums[lane >> 2] = (int16_t)gsum;
-  if (lane == 0) blk->d = 1.f / iscale;
+  const Q8KLane r = quantize_lane_q8_k(v);
+  *reinterpret_cast<uint32_t*>(blk->qs + 4 * lane) = r.q;
+  if ((lane & 3) == 0) blk->bsums[lane >> 2] = (int16_t)r.sum16;
+  if (lane == 0) blk->d = r.d;
 }
 
 // quantize_row_q8_0 (quantize.rs:37-55) of one block by the 32 lanes of a
@@ -290,6 +287,25 @@ __device__ __forceinline__ void quantize_block_q8_0(const float* __restrict__ xs
   const float id = d != 0.f ? 1.f / d : 0.f;
   blk->qs[i] = (int8_t)roundf(v * id);
   if (i == 0) blk->d = (float)(_Float16)d;
+}
+
+// The same of one block by an aligned group of 8 lanes, lane i holding
+// values 4i .. 4i+3.
+struct Q80Lane {
+  uint32_t q;
+  float d;
+};
+__device__ __forceinline__ Q80Lane quantize_lane_q8_0(const float (&v)[4]) {
+  float amax = fabsf(v[0]);
+#pragma unroll
+  for (int e = 1; e < 4; ++e) amax = fmaxf(amax, fabsf(v[e]));
+  amax = group_max<8>(amax);
+  const float d = amax / 127.f;
+  const float id = d != 0.f ? 1.f / d : 0.f;
+  Q80Lane r{0u, (float)(_Float16)d};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r.q |= (uint32_t)(uint8_t)(int8_t)roundf(v[e] * id) << (8 * e);
+  return r;
 }
 
 __global__ __launch_bounds__(256) void quantize_q8_k_kernel(const float* __restrict__ x, rv_block_q8_k* __restrict__ out,
@@ -486,16 +502,73 @@ __global__ __launch_bounds__(1024) void rmsnorm_kernel(const float* __restrict__
   }
 }
 
-// One workgroup per row: out[r] = rmsnorm(x[r], w, eps) over n values.
-__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                           float eps, int n, float* __restrict__ out) {
-  __shared__ double red[4];
-  const float* xr = x + (size_t)blockIdx.x * n;
-  float* orow = out + (size_t)blockIdx.x * n;
-  const float inv = block_inv_rms<256>(xr, n, eps, red);
-  for (int j = threadIdx.x; j < n; j += 256) {
+// A chunk's rows quantized into the batched GEMVs' operand order (PackedActs,
+// rv_quant.hpp), to Q8_K and, with Q0, to Q8_0; with NORM each row is
+// RMS-normalized first (norm.rs:18-58). blockIdx.x is the row, wave w takes
+// its blocks W blockIdx.y + w, then W * gridDim.y on. The normed row never
+// goes through memory: as separate launches (norm, then both quantizations
+// with one wave per block and four 6-step shuffle reductions) a 512-row chunk
+// of 2048 values took 7.0 + 7.6 us.
+template <bool NORM, bool Q0, int W>
+__global__ __launch_bounds__(64 * W) void quantize_rows_kernel(const float* __restrict__ x, int n_rows, int n,
+                                                               const float* __restrict__ norm_w, float eps,
+                                                               char* __restrict__ pk, char* __restrict__ p0) {
 #pragma clang fp contract(off)
-    orow[j] = xr[j] * inv * w[j];
+  typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
+  const int row = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int nb = n / 256, tile = row >> 4, a = row & 15, nt = min(16, n_rows - 16 * tile);
+  const float* xr = x + (size_t)row * n;
+  char* tk = pk + (size_t)tile * 16 * nb * kPackedKBytes;
+  char* t0 = Q0 ? p0 + (size_t)tile * 16 * nb * kPacked0Bytes : nullptr;
+  const int b0 = W * (int)blockIdx.y + wave;
+  // The wave's first block, loaded ahead of the norm's reduction.
+  f32x4a xv{}, wv{};
+  const int bc = min(b0, nb - 1);
+  xv = *reinterpret_cast<const f32x4a*>(xr + 256 * bc + 4 * lane);
+  if constexpr (NORM) wv = *reinterpret_cast<const f32x4a*>(norm_w + 256 * bc + 4 * lane);
+  float inv = 1.f;
+  if constexpr (NORM) {
+    __shared__ double red[4];
+    if (wave < 4) {  // 256 threads, in the order of rmsnorm_kernel's 256-thread form
+      double ss = 0.0;
+      for (int i = threadIdx.x; i < n; i += 256) {
+        const double v = (double)xr[i];
+        ss += v * v;
+      }
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+      if (lane == 0) red[wave] = ss;
+    }
+    __syncthreads();
+    double tot = 0.0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) tot += red[w];
+    inv = (float)(1.0 / sqrt(tot / (double)n + (double)eps));
+  }
+  for (int b = b0; b < nb; b += W * (int)gridDim.y) {
+    if (b != b0) {
+      xv = *reinterpret_cast<const f32x4a*>(xr + 256 * b + 4 * lane);
+      if constexpr (NORM) wv = *reinterpret_cast<const f32x4a*>(norm_w + 256 * b + 4 * lane);
+    }
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = NORM ? xv[e] * inv * wv[e] : xv[e];
+    // Values 4 lane .. + 3: bytes 4 (lane % 4) of piece lane / 4.
+    const Q8KLane k = quantize_lane_q8_k(v);
+    char* ub = tk + (size_t)b * nt * kPackedKBytes;
+    const int piece = lane >> 2;
+    *reinterpret_cast<uint32_t*>(ub + (piece * nt + a) * 16 + 4 * (lane & 3)) = k.q;
+    if ((lane & 3) == 0)
+      *reinterpret_cast<_Float16*>(ub + 256 * nt + ((piece & 3) * nt + a) * 8 + 2 * (piece >> 2)) =
+          (_Float16)(float)k.sum16;
+    if (lane == 0) *reinterpret_cast<float*>(ub + 288 * nt + 4 * a) = k.d;
+    if constexpr (Q0) {
+      const Q80Lane z = quantize_lane_q8_0(v);
+      char* zb = t0 + (size_t)b * nt * kPacked0Bytes;
+      const int blk = lane >> 3, i = lane & 7;  // values 4 i .. + 3 of the block: byte 4 (i % 2) of its piece i / 2
+      *reinterpret_cast<uint32_t*>(zb + ((4 * (blk >> 1) + (i >> 1)) * nt + a) * 16 + 8 * (blk & 1) + 4 * (i & 1)) = z.q;
+      if (i == 0) *reinterpret_cast<float*>(zb + 256 * nt + 32 * a + 4 * blk) = z.d;
+    }
   }
 }
 
@@ -518,362 +591,6 @@ void launch_rows_t(const uint8_t* w, size_t row_bytes, int nb, const void* acts,
 }
 
 
-// ---- batched GEMV on int8 MFMA (gemv.rs:444-543, :616-651) ------------------
-//
-// out[i][a] = row(row_lo + i) . act_row(a) for a tile of 32 weight rows x
-// 32 * W activation rows (one 32-row tile per wave) per workgroup. Every output is the
-// scalar dot's f32 value bit for bit: the integer sums are exact (int8
-// products, int32 accumulation) and the per-block float expression and the
-// block order are the scalar kernel's.
-//
-// The k-quant integer sums go through v_mfma_i32_32x32x32_i8 with the
-// sub-block scales folded into the weights (the A operand, weight rows =
-// the MFMA's rows; the activations' int8 values are B, one column per
-// activation row). sc * q does not fit in int8; the scale is split instead,
-// so that each plane is a packed product with no carries between bytes:
-//   Q4_K: sc = 8 sh + sl (sh, sl <= 7), q <= 15: planes sh*q, sl*q (<= 105)
-//     and the mins m broadcast over their sub-block: sumi = 8 H + L,
-//     sumi_mins = M (the Q8_K bsums are exactly the sub-block sums of the
-//     activation values);
-//   Q5_K: the same on q - 16 (sh*(q-16) in [-112, 105]) plus the scales
-//     broadcast: sumi = 8 H + L + 16 S, sumi_mins = M;
-//   Q6_K: sum_s sc_s (sum q a - 32 bsum_s) (dot.rs:150-179) is exactly
-//     sum sc (q - 32) a; sc (q - 32) = 64 hi + lo (lo < 64): sumi = 64 H + L;
-//   Q8_0: the weight bytes themselves, one MFMA per 32-weight block.
-// The planes of one block (eight Q8_0 blocks) of the workgroup's 32 rows
-// are built once in LDS, one thread per (row, 32-weight sub-block), and
-// used by every activation tile of the workgroup.
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int kBRows = 32;
-constexpr int kPlaneRow = 272;  // 256 bytes + 16: 16-byte LDS reads of 32 rows spread over the banks
-
-struct BatchedArgs {
-  const uint8_t* w;
-  size_t row_bytes;
-  int nb;            // weight blocks per row (k-quant: 256 weights, Q8_0: 32)
-  const void* acts;  // n_acts rows of nb Q8_K (k-quants) or Q8_0 blocks
-  int n_acts;
-  long row_lo;
-  int n_rows;
-  float* out;
-  long ldo;
-  int transposed;    // 0: out[i * ldo + a] (the reference's layout); 1: out[a * ldo + i]
-  int accumulate;    // out += dot (one f32 add, as the prefill's residual add)
-};
-
-__device__ __forceinline__ uint32_t pack4(int a, int b, int c, int d) {
-  return (uint32_t)(a & 0xFF) | ((uint32_t)(b & 0xFF) << 8) | ((uint32_t)(c & 0xFF) << 16) | ((uint32_t)d << 24);
-}
-
-// 32 bytes at a 2-byte-aligned address as raw dwords (aligned-down reads
-// plus a 2-byte tail, as load32_a2), with the realignment left to
-// fix32_a2, so the loads can be issued one step ahead of their use.
-struct Raw32 {
-  uint32_t e[8];
-  uint32_t tail;
-  bool odd;
-};
-__device__ __forceinline__ Raw32 raw32_a2(const uint8_t* a) {
-  Raw32 r;
-  r.odd = ((uintptr_t)a & 2) != 0;
-  const uint32_t* p = reinterpret_cast<const uint32_t*>(a - (r.odd ? 2 : 0));
-#pragma unroll
-  for (int k = 0; k < 8; ++k) r.e[k] = p[k];
-  r.tail = r.odd ? *reinterpret_cast<const uint16_t*>(a + 30) : 0u;
-  return r;
-}
-__device__ __forceinline__ void fix32_a2(const Raw32& r, uint32_t (&w)[8]) {
-#pragma unroll
-  for (int k = 0; k < 7; ++k) w[k] = r.odd ? __builtin_amdgcn_alignbyte(r.e[k + 1], r.e[k], 2) : r.e[k];
-  w[7] = r.odd ? (r.e[7] >> 16) | (r.tail << 16) : r.e[7];
-}
-
-// The bytes thread (r, j) needs to build its row's sub-block j of one block
-// (or block j of a group of eight Q8_0 blocks), loaded one step ahead.
-template <int FMT>
-struct WRaw {
-  uint32_t hdr[4];  // k-quants: d/dmin dword and the 12 scale bytes; Q6_K: scale pair, d
-  uint32_t q[8];    // Q4_K/Q5_K quants
-  uint32_t h[8];    // Q5_K high bits
-  Raw32 a, b;       // Q6_K ql / qh; Q8_0 qs (a) and d (hdr[0])
-};
-
-template <int FMT>
-__device__ __forceinline__ void load_wraw(const uint8_t* __restrict__ blk, int j, WRaw<FMT>& w) {
-  if constexpr (FMT == RV_QF_Q4_K || FMT == RV_QF_Q5_K) {
-    constexpr bool kQ5 = FMT == RV_QF_Q5_K;
-    const uint32_t* hp = reinterpret_cast<const uint32_t*>(blk);
-    w.hdr[0] = hp[0], w.hdr[1] = hp[1], w.hdr[2] = hp[2], w.hdr[3] = hp[3];
-    const u32x4a* qp = reinterpret_cast<const u32x4a*>(blk + (kQ5 ? 48 : 16) + 32 * (j >> 1));
-    const u32x4a q0 = qp[0], q1 = qp[1];
-    w.q[0] = q0[0], w.q[1] = q0[1], w.q[2] = q0[2], w.q[3] = q0[3];
-    w.q[4] = q1[0], w.q[5] = q1[1], w.q[6] = q1[2], w.q[7] = q1[3];
-    if constexpr (kQ5) {
-      const u32x4a* qh = reinterpret_cast<const u32x4a*>(blk + 16);
-      const u32x4a h0 = qh[0], h1 = qh[1];
-      w.h[0] = h0[0], w.h[1] = h0[1], w.h[2] = h0[2], w.h[3] = h0[3];
-      w.h[4] = h1[0], w.h[5] = h1[1], w.h[6] = h1[2], w.h[7] = h1[3];
-    }
-  } else if constexpr (FMT == RV_QF_Q6_K) {
-    const int half = j >> 2, grp = j & 3;
-    w.a = raw32_a2(blk + 64 * half + 32 * (grp & 1));
-    w.b = raw32_a2(blk + 128 + 32 * half);
-    w.hdr[0] = *reinterpret_cast<const uint16_t*>(blk + 192 + 2 * j);
-    w.hdr[1] = *reinterpret_cast<const uint16_t*>(blk + 208);
-  } else {
-    w.a = raw32_a2(blk + 2);
-    w.hdr[0] = *reinterpret_cast<const uint16_t*>(blk);
-  }
-}
-
-// Thread (r, j) writes the 32 plane bytes of its row's sub-block j
-// (weights 32j .. 32j+31 of the block) and, for j == 0, the row's block
-// scalars (Q8_0: block j's d).
-template <int FMT>
-__device__ __forceinline__ void build_planes(const WRaw<FMT>& wr, int j, int8_t (*pl)[kBRows][kPlaneRow], int r,
-                                             float (*sd)[kBRows]) {
-  uint32_t q[8];
-  int sc[2], m = 0;
-  if constexpr (FMT == RV_QF_Q4_K || FMT == RV_QF_Q5_K) {
-    const uint32_t s3[3] = {wr.hdr[1], wr.hdr[2], wr.hdr[3]};
-    scale_min_k4(j, s3, sc[0], m);
-    sc[1] = sc[0];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      q[k] = (j & 1) ? (wr.q[k] >> 4) & 0x0F0F0F0Fu : wr.q[k] & 0x0F0F0F0Fu;
-      if constexpr (FMT == RV_QF_Q5_K) q[k] |= ((wr.h[k] >> j) & 0x01010101u) << 4;
-    }
-    if (j == 0) {
-      sd[0][r] = f16_bits_to_f32(wr.hdr[0]);
-      sd[1][r] = f16_bits_to_f32(wr.hdr[0] >> 16);
-    }
-  } else if constexpr (FMT == RV_QF_Q6_K) {
-    const int grp = j & 3;
-    uint32_t ql[8], qh[8];
-    fix32_a2(wr.a, ql);
-    fix32_a2(wr.b, qh);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const uint32_t nib = (grp >> 1) ? (ql[k] >> 4) & 0x0F0F0F0Fu : ql[k] & 0x0F0F0F0Fu;
-      q[k] = nib | (((qh[k] >> (2 * grp)) & 0x03030303u) << 4);
-    }
-    sc[0] = (int)(int8_t)(wr.hdr[0] & 0xFF);
-    sc[1] = (int)(int8_t)(wr.hdr[0] >> 8);
-    if (j == 0) sd[0][r] = f16_bits_to_f32(wr.hdr[1]);
-  } else {
-    fix32_a2(wr.a, q);
-    sd[j][r] = f16_bits_to_f32(wr.hdr[0]);
-  }
-  auto plane = [&](int p) { return reinterpret_cast<u32x4a*>(&pl[p][r][32 * j]); };
-  auto put = [&](int p, const uint32_t (&v)[8]) {
-    plane(p)[0] = u32x4a{v[0], v[1], v[2], v[3]};
-    plane(p)[1] = u32x4a{v[4], v[5], v[6], v[7]};
-  };
-  if constexpr (FMT == RV_QF_Q8_0) {
-    put(0, q);
-  } else if constexpr (FMT == RV_QF_Q4_K || FMT == RV_QF_Q5_K) {
-    // q bytes times a 3-bit scale part: four exact byte products per dword.
-    const uint32_t sh = (uint32_t)sc[0] >> 3, sl = (uint32_t)sc[0] & 7;
-    uint32_t h[8], l[8], mm[8], ss[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      if constexpr (FMT == RV_QF_Q4_K) {
-        h[k] = q[k] * sh;
-        l[k] = q[k] * sl;
-      } else {
-        // bytes s*q + (128 - 16 s) in [16, 233] (no carries), then the top
-        // bit flipped: the signed bytes s*(q - 16).
-        h[k] = (q[k] * sh + (128u - 16u * sh) * 0x01010101u) ^ 0x80808080u;
-        l[k] = (q[k] * sl + (128u - 16u * sl) * 0x01010101u) ^ 0x80808080u;
-        ss[k] = (uint32_t)sc[0] * 0x01010101u;
-      }
-      mm[k] = (uint32_t)m * 0x01010101u;
-    }
-    put(0, h);
-    put(1, l);
-    put(2, mm);
-    if constexpr (FMT == RV_QF_Q5_K) put(3, ss);
-  } else {
-    uint32_t h[8], l[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int s2 = sc[k >> 2];  // the first 16 weights take sc[0], the rest sc[1]
-      int hi[4], lo[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int v = s2 * ((int)((q[k] >> (8 * e)) & 0xFF) - 32);
-        hi[e] = v >> 6;  // arithmetic shift: floor, so lo = v - 64 hi is in [0, 64)
-        lo[e] = v & 63;
-      }
-      h[k] = pack4(hi[0], hi[1], hi[2], hi[3]);
-      l[k] = pack4(lo[0], lo[1], lo[2], lo[3]);
-    }
-    put(0, h);
-    put(1, l);
-  }
-}
-
-// The activation operands of one step for one tile: lane (li, kh) holds
-// activation row li's bytes 16 kh .. 16 kh + 15 of each 32-value chunk.
-template <bool Q80>
-__device__ __forceinline__ void load_acts(const void* __restrict__ acts, int act, int nb, int step, i32x4 (&bq)[8],
-                                          float (&da)[8], int kh) {
-  if constexpr (Q80) {
-    const rv_block_q8_0* y = reinterpret_cast<const rv_block_q8_0*>(acts) + (size_t)act * nb;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const rv_block_q8_0* yb = y + min(8 * step + c, nb - 1);
-      const u32x4a v = *reinterpret_cast<const u32x4a*>(yb->qs + 16 * kh);
-      bq[c] = i32x4{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
-      da[c] = yb->d;
-    }
-  } else {
-    const rv_block_q8_k* y = reinterpret_cast<const rv_block_q8_k*>(acts) + (size_t)act * nb + step;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const u32x4a v = *reinterpret_cast<const u32x4a*>(y->qs + 32 * c + 16 * kh);
-      bq[c] = i32x4{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
-    }
-    da[0] = y->d;
-  }
-}
-
-template <int FMT, int W>
-__global__ __launch_bounds__(64 * W) void gemv_batched_kernel(BatchedArgs a) {
-#pragma clang fp contract(off)
-  constexpr bool kQ80 = FMT == RV_QF_Q8_0;
-  constexpr int kPlanes = kQ80 ? 1 : FMT == RV_QF_Q6_K ? 2 : FMT == RV_QF_Q5_K ? 4 : 3;
-  constexpr int BB = FMT == RV_QF_Q4_K ? 144 : FMT == RV_QF_Q5_K ? 176 : FMT == RV_QF_Q6_K ? 210 : 34;
-  constexpr int NB = 4 / W;  // (row, sub-block) build tasks per thread: 256 per step
-  __shared__ __attribute__((aligned(16))) int8_t pl[kPlanes][kBRows][kPlaneRow];
-  // Per-row block scalars, row-minor so a lane's four consecutive output
-  // rows come in one 16-byte read: k-quants [0] d and [1] dmin; Q8_0 [c]
-  // the d of block c of the group.
-  __shared__ __attribute__((aligned(16))) float sd[8][kBRows];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, kh = lane >> 5;
-  const int row0 = blockIdx.x * kBRows;
-  // Builder role: task u = tid + 64 W n -> (row u >> 3, sub-block u & 7);
-  // rows past the range re-read the last row (their outputs are not stored).
-  const uint8_t* wrow[NB];
-#pragma unroll
-  for (int n = 0; n < NB; ++n)
-    wrow[n] = a.w + (size_t)(a.row_lo + min(row0 + ((tid + 64 * W * n) >> 3), a.n_rows - 1)) * a.row_bytes;
-  const int bj = tid & 7;  // the same for every task of the thread (64 W is a multiple of 8)
-  auto wblk = [&](int n, int step) {
-    return kQ80 ? wrow[n] + (size_t)min(8 * step + bj, a.nb - 1) * BB : wrow[n] + (size_t)step * BB;
-  };
-  const int act = min((int)blockIdx.y * 32 * W + 32 * wave + li, a.n_acts - 1);
-  float sumf[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) sumf[r] = 0.f;
-  const int n_steps = kQ80 ? (a.nb + 7) / 8 : a.nb;
-  // Software pipeline: the weight bytes of steps + 1 .. + 2 and the
-  // activation operands of step + 1 are in flight while step's planes are
-  // built and its MFMAs run (a weight block's memory round trip is longer
-  // than one step). The register rings are indexed by the unrolled u. Every
-  // load is issued unconditionally (steps past the end re-read the last
-  // one): a conditional load would make the compiler merge the old and new
-  // registers after the branch and wait for the load right there.
-  constexpr int DW = 3, DA = 2;
-  const int last = n_steps - 1;
-  WRaw<FMT> wr[DW][NB];
-#pragma unroll
-  for (int u = 0; u < DW; ++u)
-#pragma unroll
-    for (int n = 0; n < NB; ++n) load_wraw<FMT>(wblk(n, min(u, last)), bj, wr[u][n]);
-  i32x4 bq[DA][8];
-  float da[DA][8];
-#pragma unroll
-  for (int u = 0; u < DA; ++u) load_acts<kQ80>(a.acts, act, a.nb, min(u, last), bq[u], da[u], kh);
-  for (int s0 = 0; s0 < n_steps; s0 += DW * DA) {
-#pragma unroll
-  for (int u = 0; u < DW * DA; ++u) {
-    const int step = s0 + u;
-    if (step >= n_steps) break;
-    const int uw = u % DW, ua = u % DA;
-#pragma unroll
-    for (int n = 0; n < NB; ++n) build_planes<FMT>(wr[uw][n], bj, pl, (tid + 64 * W * n) >> 3, sd);
-    __syncthreads();
-#pragma unroll
-    for (int n = 0; n < NB; ++n) load_wraw<FMT>(wblk(n, min(step + DW, last)), bj, wr[uw][n]);
-    i32x4 cur[8];
-    float dcur[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) cur[c] = bq[ua][c], dcur[c] = da[ua][c];
-    load_acts<kQ80>(a.acts, act, a.nb, min(step + DA, last), bq[ua], da[ua], kh);
-    // Lane (li, kh) owns output rows 8 g + 4 kh + e (e < 4) of the tile, g < 4.
-    auto rows4 = [&](int k, int g) { return *reinterpret_cast<const f32x4*>(&sd[k][8 * g + 4 * kh]); };
-    auto aop = [&](int p, int c) { return *reinterpret_cast<const i32x4*>(&pl[p][li][32 * c + 16 * kh]); };
-    if constexpr (kQ80) {
-      const int nblk = min(8, a.nb - 8 * step);
-      i32x4 wa = aop(0, 0);
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        i32x16 acc = {};
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(wa, cur[c], acc, 0, 0, 0);
-        if (c + 1 < 8) wa = aop(0, c + 1);  // in flight under this MFMA
-        f32x4 dw[4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) dw[g] = rows4(c, g);
-        if (c < nblk) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) sumf[r] += (float)acc[r] * (dw[r >> 2][r & 3] * dcur[c]);
-        }
-      }
-    } else {
-      f32x4 dw[4], dm[4];
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        dw[g] = rows4(0, g);
-        if constexpr (FMT != RV_QF_Q6_K) dm[g] = rows4(1, g);
-      }
-      i32x16 acc[kPlanes];
-#pragma unroll
-      for (int p = 0; p < kPlanes; ++p) acc[p] = i32x16{};
-      i32x4 wa[kPlanes], wn[kPlanes];
-#pragma unroll
-      for (int p = 0; p < kPlanes; ++p) wa[p] = aop(p, 0);
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        if (c + 1 < 8) {
-#pragma unroll
-          for (int p = 0; p < kPlanes; ++p) wn[p] = aop(p, c + 1);  // in flight under chunk c's MFMAs
-        }
-#pragma unroll
-        for (int p = 0; p < kPlanes; ++p) acc[p] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wa[p], cur[c], acc[p], 0, 0, 0);
-#pragma unroll
-        for (int p = 0; p < kPlanes; ++p) wa[p] = wn[p];
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float dr = dw[r >> 2][r & 3];
-        if constexpr (FMT == RV_QF_Q6_K) {
-          const int sumi = 64 * acc[0][r] + acc[1][r];
-          sumf[r] += dr * dcur[0] * (float)sumi;
-        } else {
-          int sumi = 8 * acc[0][r] + acc[1][r];
-          if constexpr (FMT == RV_QF_Q5_K) sumi += 16 * acc[3][r];
-          const float d = dr * dcur[0], dmin = dm[r >> 2][r & 3] * dcur[0];
-          sumf[r] += d * (float)sumi - dmin * (float)acc[2][r];
-        }
-      }
-    }
-    __syncthreads();  // the next step's planes overwrite these
-  }
-  }
-  const int act_out = (int)blockIdx.y * 32 * W + 32 * wave + li;
-  if (act_out >= a.n_acts) return;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int i = row0 + 8 * (r >> 2) + 4 * kh + (r & 3);
-    if (i < a.n_rows) {
-      float* o = a.out + (a.transposed ? (size_t)act_out * a.ldo + i : (size_t)i * a.ldo + act_out);
-      *o = a.accumulate ? *o + sumf[r] : sumf[r];
-    }
-  }
-}
 }  // namespace
 
 HipStatus launch_quantize_q8_k(const float* x, rv_block_q8_k* out, size_t n_blocks, hipStream_t s) {
@@ -953,49 +670,23 @@ HipStatus launch_vec_add(float* a, const float* b, size_t n, hipStream_t s) {
   return st;
 }
 
-template <int FMT, int W>
-void launch_batched_t(const BatchedArgs& a, hipStream_t s) {
-  const dim3 grid((unsigned)((a.n_rows + kBRows - 1) / kBRows), (unsigned)((a.n_acts + 32 * W - 1) / (32 * W)));
-  hipLaunchKernelGGL((gemv_batched_kernel<FMT, W>), grid, dim3(64 * W), 0, s, a);
-}
-
-template <int FMT>
-void launch_batched_f(const BatchedArgs& a, hipStream_t s) {
-  // Four 32-activation tiles per workgroup share its planes; Q8_0 matrices
-  // with few row tiles (the k projection: 16) take one tile per workgroup
-  // instead, four times the workgroups (its plane build is a copy).
-  const long row_tiles = (a.n_rows + kBRows - 1) / kBRows;
-  if (FMT == RV_QF_Q8_0 && row_tiles * ((a.n_acts + 127) / 128) < 256)
-    launch_batched_t<FMT, 1>(a, s);
+HipStatus launch_quantize_rows(const float* x, size_t n_rows, size_t n, const float* norm_w, float eps, void* packed_k,
+                               void* packed_0, hipStream_t s) {
+  HipStatus st;
+  if (n_rows == 0 || n == 0) return st;
+  char *pk = (char*)packed_k, *p0 = (char*)packed_0;
+  const unsigned nb = (unsigned)(n / 256);
+  if (norm_w)
+    hipLaunchKernelGGL((quantize_rows_kernel<true, true, 8>), dim3((unsigned)n_rows), dim3(512), 0, s, x, (int)n_rows,
+                       (int)n, norm_w, eps, pk, p0);
+  else if (p0)
+    hipLaunchKernelGGL((quantize_rows_kernel<false, true, 4>), dim3((unsigned)n_rows, (nb + 3) / 4), dim3(256), 0, s, x,
+                       (int)n_rows, (int)n, norm_w, eps, pk, p0);
   else
-    launch_batched_t<FMT, 4>(a, s);
-}
-
-HipStatus launch_gemv_batched(uint32_t fmt, const uint8_t* w, size_t row_bytes, size_t in_dim, const void* acts,
-                              size_t n_acts, size_t row_lo, size_t n_rows, float* out, size_t ldo, bool transposed,
-                              hipStream_t s, bool accumulate) {
-  HipStatus st;
-  if (n_rows == 0 || n_acts == 0) return st;
-  BatchedArgs a{w, row_bytes, (int)(in_dim / (fmt == RV_QF_Q8_0 ? 32 : 256)), acts, (int)n_acts, (long)row_lo,
-                (int)n_rows, out, (long)ldo, transposed ? 1 : 0, accumulate ? 1 : 0};
-  switch (fmt) {
-    case RV_QF_Q4_K: launch_batched_f<RV_QF_Q4_K>(a, s); break;
-    case RV_QF_Q5_K: launch_batched_f<RV_QF_Q5_K>(a, s); break;
-    case RV_QF_Q6_K: launch_batched_f<RV_QF_Q6_K>(a, s); break;
-    default: launch_batched_f<RV_QF_Q8_0>(a, s);
-  }
+    hipLaunchKernelGGL((quantize_rows_kernel<false, false, 4>), dim3((unsigned)n_rows, (nb + 3) / 4), dim3(256), 0, s,
+                       x, (int)n_rows, (int)n, norm_w, eps, pk, p0);
   st.e = hipGetLastError();
-  if (st.e != hipSuccess) st.what = "batched gemv launch";
-  return st;
-}
-
-HipStatus launch_rmsnorm_rows(const float* x, const float* w, float eps, size_t n_rows, size_t n, float* out,
-                              hipStream_t s) {
-  HipStatus st;
-  if (n_rows == 0) return st;
-  hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)n_rows), dim3(256), 0, s, x, w, eps, (int)n, out);
-  st.e = hipGetLastError();
-  if (st.e != hipSuccess) st.what = "rmsnorm rows launch";
+  if (st.e != hipSuccess) st.what = "quantize rows launch";
   return st;
 }
 

@@ -95,9 +95,52 @@ int32_t in_proj_rows_check(InProj& p, size_t n_rows, size_t wq_len, size_t wk_le
 int32_t out_proj_rows_check(OutProj& p, size_t n_rows, size_t wo_len, rv_error* err);
 HipStatus in_proj_rows_launch(const InProj& p, size_t n_rows, hipStream_t s);
 HipStatus out_proj_rows_launch(const OutProj& p, size_t n_rows, hipStream_t s);
-// out[r] = rmsnorm(x[r], w, eps), n_rows rows of n values.
-HipStatus launch_rmsnorm_rows(const float* x, const float* w, float eps, size_t n_rows, size_t n, float* out,
-                              hipStream_t s);
+
+// PackedActs: a chunk's quantized rows in the batched GEMVs' operand order.
+// Tile t holds rows 16 t .. + nt (nt = 16, or what is left) and starts after
+// the whole tiles before it; within it one unit per 256-value block,
+// kPackedKBytes * nt (Q8_K) or kPacked0Bytes * nt (Q8_0) bytes, no larger
+// than the rows' block structs. Row a of the tile has, in a unit:
+//  - 16 pieces of 16 quants: piece i at (i * nt + a) * 16. Q8_K: values 16 i
+//    .. + 15. Q8_0: piece 4 c + kq is values 8 kq .. + 7 of block 2 c and the
+//    same of block 2 c + 1;
+//  - Q8_K: at 256 nt + (kq * nt + a) * 8 the sums of pieces kq, 4 + kq, 8 + kq
+//    and 12 + kq as f16 (at most 2048 in magnitude: exact), and at 288 nt +
+//    4 a the scale d; Q8_0: at 256 nt + 32 a the eight blocks' d.
+constexpr int kPackedKBytes = 292, kPacked0Bytes = 288;
+static_assert(kPackedKBytes == sizeof(rv_block_q8_k) && kPacked0Bytes == 8 * sizeof(rv_block_q8_0), "packed unit sizes");
+// n_rows rows of n values (a multiple of 256) into packed_k and, unless null,
+// packed_0; with norm_w each row is RMS-normalized first (both forms then).
+HipStatus launch_quantize_rows(const float* x, size_t n_rows, size_t n, const float* norm_w, float eps, void* packed_k,
+                               void* packed_0, hipStream_t s);
+
+// The batched GEMVs (rv_batched.hip): up to three matrices over the same
+// activation rows in one launch.
+struct BatchedSeg {
+  uint32_t fmt;
+  const uint8_t* w;
+  size_t row_bytes;
+  long row_lo;
+  int n_rows;
+  float* out;
+  long ldo;
+  // Filled by launch_batched: row groups and workgroups.
+  int n_rg, blocks;
+};
+struct BatchedArgs {
+  int n_seg;
+  BatchedSeg seg[3];
+  const void* acts_k;  // n_acts rows of in_dim / 256 Q8_K units (blocks when not packed), for the k-quants
+  const void* acts_0;  // the same in Q8_0
+  int n_acts;
+  int in_dim;
+  int transposed;  // 0: out[i * ldo + a] (the reference's layout); 1: out[a * ldo + i]
+  int accumulate;  // out += dot (one f32 add, as the prefill's residual add)
+  int n_ag;        // activation groups (filled by launch_batched)
+};
+// out = row(row_lo + i) . act_row(a) for every segment, i < n_rows, a <
+// n_acts; in_dim > 0, and a multiple of 256 when packed.
+HipStatus launch_batched(BatchedArgs a, bool packed, hipStream_t s);
 
 HipStatus launch_quantize_q8_k(const float* x, rv_block_q8_k* out, size_t n_blocks, hipStream_t s);
 HipStatus launch_quantize_q8_0(const float* x, rv_block_q8_0* out, size_t n_blocks, hipStream_t s);
@@ -110,13 +153,6 @@ HipStatus launch_quantize_both(const float* x, rv_block_q8_k* ok, rv_block_q8_0*
 HipStatus launch_gemv_rows(uint32_t fmt, const uint8_t* w, size_t row_bytes, size_t in_dim, const void* acts,
                            size_t row_lo, size_t n_rows, float* out, hipStream_t s);
 HipStatus launch_fused_proj(const FusedProjArgs& a, hipStream_t s);
-// Batched GEMV (int8 MFMA): out[i * ldo + a] (or, transposed, out[a * ldo + i])
-// = row(row_lo + i) . act_row(a), i < n_rows, a < n_acts; acts holds n_acts
-// rows of in_dim / 256 Q8_K (or in_dim / 32 Q8_0 for RV_QF_Q8_0) blocks.
-// in_dim > 0. With accumulate, out += the dot instead.
-HipStatus launch_gemv_batched(uint32_t fmt, const uint8_t* w, size_t row_bytes, size_t in_dim, const void* acts,
-                              size_t n_acts, size_t row_lo, size_t n_rows, float* out, size_t ldo, bool transposed,
-                              hipStream_t s, bool accumulate = false);
 // out = rmsnorm(x, w, eps) over n values (one workgroup; norm.rs:38-58).
 HipStatus launch_rmsnorm(const float* x, const float* w, float eps, size_t n, float* out, hipStream_t s);
 // a[i] += b[i], i < n (vec.rs:10-22).

@@ -178,3 +178,31 @@ def test_prefill_chunk_projections_match_the_single_row_gemvs(n):
         assert v[r].tobytes() == oracle.gemv(Q.RV_QF_Q6_K, wv, hidden, kv_dim, ak).tobytes(), f"v row {r}"
         o = oracle.gemv(Q.RV_QF_Q5_K, wo, q_dim, hidden, oracle.quantize_row_q8_k(attn[r]))
         assert r_got[r].tobytes() == (res[r] + o).astype(F32).tobytes(), f"residual row {r}"
+
+
+@pytest.mark.parametrize("q_fmt,v_fmt", [(oracle.RV_QF_Q5_K, oracle.RV_QF_Q6_K), (oracle.RV_QF_Q6_K, oracle.RV_QF_Q4_K),
+                                         (oracle.RV_QF_Q4_K, oracle.RV_QF_Q5_K)])
+@pytest.mark.parametrize("n,blocks", [(1, 1), (15, 4), (16, 5), (17, 3), (129, 9)])
+def test_rows_projections_at_tile_edges(q_fmt, v_fmt, n, blocks):
+    """The rows forms around 16-row activation tiles, 128-row workgroups,
+    16-row weight tiles (dims 40 and 17) and chunks of four blocks, with rows
+    that are zero, constant, tied in magnitude or hold one large value."""
+    torch = torch_cuda()
+    Q = oracle
+    hidden, q_dim, kv_dim = 256 * blocks, 40, 17
+    rng = np.random.default_rng(0xED6E + 64 * n + blocks + q_fmt)
+    wq, wk, wv = (random_weight_rows(f, m, hidden, rng)
+                  for f, m in ((q_fmt, q_dim), (Q.RV_QF_Q8_0, kv_dim), (v_fmt, kv_dim)))
+    x = rng.standard_normal((n, hidden)).astype(F32)
+    x[0, :256] = 0.0
+    x[n // 2] = -3.0 if n > 2 else x[n // 2]
+    x[n - 1, 5], x[n - 1, 133] = 60.0, -60.0
+    say(f"case rows projections q={q_fmt} v={v_fmt} n={n} blocks={blocks}")
+    q, k, v = (torch.full((n, m), float("nan"), device="cuda") for m in (q_dim, kv_dim, kv_dim))
+    P.attn_in_proj_rows(torch.from_numpy(x).cuda(), q_fmt, dev_u8(torch, wq), q, dev_u8(torch, wk), k, v_fmt,
+                        dev_u8(torch, wv), v)
+    torch.cuda.synchronize()
+    ak, a0 = quantize_rows(Q.RV_QF_Q4_K, x), quantize_rows(Q.RV_QF_Q8_0, x)
+    for got, fmt, w, m, acts in ((q, q_fmt, wq, q_dim, ak), (k, Q.RV_QF_Q8_0, wk, kv_dim, a0), (v, v_fmt, wv, kv_dim, ak)):
+        want = oracle.gemv(fmt, w, hidden, m, acts, n_acts=n, rows=(0, m)).reshape(m, n).T
+        assert got.cpu().numpy().tobytes() == np.ascontiguousarray(want).tobytes(), f"fmt {fmt}"
