@@ -63,3 +63,24 @@ def test_router_validation_order():
     with pytest.raises(rv.RamvampError) as ei:
         R.router_topk(x, torch.ones(4, 7, device="cuda").reshape(4, 7)[:, :7].contiguous(), 2, False)
     assert ei.value.variant in ("LengthMismatch",)
+
+
+@pytest.mark.parametrize("n_rows,hidden,n_experts,top_k", [(1, 64, 1, 1), (2, 128, 64, 64), (3, 192, 65, 65),
+                                                           (1, 256, 128, 128), (257, 448, 127, 3), (601, 320, 17, 5)])
+def test_router_staged_form_at_its_edges(n_rows, hidden, n_experts, top_k):
+    """One to seven 64-value chunks (the ring of three and its remainders),
+    experts around the two sum waves, every expert chosen, a ragged last group
+    of 2 and of 4 rows; a row of zeros, tied experts, infinite and NaN logits."""
+    torch = torch_cuda()
+    say(f"case router staged rows={n_rows} hidden={hidden} experts={n_experts} top_k={top_k}")
+    rng = np.random.default_rng(hidden * n_experts + n_rows)
+    x = rng.standard_normal((n_rows, hidden)).astype(np.float32)
+    router = (rng.standard_normal((n_experts, hidden)) * 0.05).astype(np.float32)
+    router[n_experts // 2] = router[0]  # a tie across the lanes
+    x[n_rows - 1] = 0.0
+    check(torch, x, router, top_k, True)
+    x[0, 3] = np.inf  # logits of either infinity (and NaN where the weight is 0)
+    router[n_experts - 1, 3] = 0.0
+    check(torch, x, router, top_k, False)
+    x[0, 3] = np.nan
+    check(torch, x, router, top_k, False)
