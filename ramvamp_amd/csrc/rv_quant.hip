@@ -265,14 +265,17 @@ __device__ __forceinline__ Q8KLane quantize_lane_q8_k(const float (&v)[4]) {
   return r;
 }
 
+__device__ __forceinline__ void store_q8_k(const Q8KLane& r, rv_block_q8_k* blk, int lane) {
+  *reinterpret_cast<uint32_t*>(blk->qs + 4 * lane) = r.q;
+  if ((lane & 3) == 0) blk->bsums[lane >> 2] = (int16_t)r.sum16;
+  if (lane == 0) blk->d = r.d;
+}
+
 __device__ __forceinline__ void quantize_block_q8_k(const float* __restrict__ xs, rv_block_q8_k* blk, int lane) {
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = xs[4 * lane + e];
-  const Q8KLane r = quantize_lane_q8_k(v);
-  *reinterpret_cast<uint32_t*>(blk->qs + 4 * lane) = r.q;
-  if ((lane & 3) == 0) blk->bsums[lane >> 2] = (int16_t)r.sum16;
-  if (lane == 0) blk->d = r.d;
+  store_q8_k(quantize_lane_q8_k(v), blk, lane);
 }
 
 // quantize_row_q8_0 (quantize.rs:37-55) of one block by the 32 lanes of a
@@ -395,10 +398,26 @@ __device__ __forceinline__ float block_inv_rms(const float* __restrict__ x, int 
   return (float)(1.0 / sqrt(tot / (double)n + (double)eps));
 }
 
-template <bool NORM>
+// Sum over the wave in the order of a shuffle tree over lanes 32, 16, .., 1
+// apart, by swaps and DPP (after the first three steps the values repeat every
+// eight lanes, so a rotation by 4 reaches the lane 4 apart).
+__device__ __forceinline__ double wave_sum_tree_f64(double x) {
+  x = swap_sum_f64<32>(x);
+  x = swap_sum_f64<16>(x);
+  x += dpp_f64<0x128>(x);  // row_ror:8
+  x += dpp_f64<0x124>(x);  // row_ror:4
+  x += dpp_f64<DPP_QUAD_XOR2>(x);
+  x += dpp_f64<DPP_QUAD_XOR1>(x);
+  return x;
+}
+
+// NB: Q8_K blocks per wave (x holds at most 256 * kFusedWaves * NB values).
+template <bool NORM, int NB>
 __global__ __launch_bounds__(64 * kFusedWaves) void fused_proj_kernel(FusedProjArgs a) {
-  __shared__ rv_block_q8_k lk[kFusedMaxKBlocks];
-  __shared__ rv_block_q8_0 l0[kFusedMax0Blocks];
+#pragma clang fp contract(off)
+  typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
+  __shared__ rv_block_q8_k lk[kFusedWaves * NB];
+  __shared__ rv_block_q8_0 l0[kFusedWaves * NB * 8];
   // The wave index as a scalar: the row, its segment and the segment's
   // fields are then wave-uniform, read with scalar loads from the kernel
   // arguments (indexed from a vector register, each was a vector load of
@@ -406,6 +425,24 @@ __global__ __launch_bounds__(64 * kFusedWaves) void fused_proj_kernel(FusedProjA
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (a.gate_pos && *a.gate_pos > a.gate_max) return;  // the whole grid: its decode step was refused
   const int first = (int)blockIdx.x * kFusedWaves;
+  // The lane's four values of each of the wave's blocks (blocks past the row
+  // re-read its last), straight into the quantizers' registers; with the norm
+  // also its weight and, for the sum of squares, the values in the summing
+  // order (thread t: t, t + 512, ..).
+  f32x4a xv[NB], wv[NB];
+  float xs[NORM ? 4 * NB : 1];
+  const int n = a.nbk * 256;
+  if constexpr (NORM) {
+#pragma unroll
+    for (int r = 0; r < 4 * NB; ++r) xs[r] = a.x[min((int)threadIdx.x + 64 * kFusedWaves * r, n - 1)];
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int at = 256 * min(wave + kFusedWaves * i, a.nbk - 1) + 4 * lane;
+    xv[i] = *reinterpret_cast<const f32x4a*>(a.x + at);
+    if constexpr (NORM) wv[i] = *reinterpret_cast<const f32x4a*>(a.norm_w + at);
+  }
+  asm volatile("" ::: "memory");  // the row loads above issue first
   // The segments this workgroup's rows touch decide which forms it needs.
   bool need_k = false, need_0 = false;
   {
@@ -422,66 +459,49 @@ __global__ __launch_bounds__(64 * kFusedWaves) void fused_proj_kernel(FusedProjA
   // one dword from each of its 128-byte lines (lane l: byte 128 l, clamped
   // to the row and aligned down; the matrix base is 4-byte aligned, so the
   // address stays inside it). The value is consumed only after the barrier,
-  // so nothing waits for it. With the norm it is issued after the loads of
-  // x and the norm weight, which the norm waits for first (loads retire in
-  // order).
+  // so nothing waits for it.
   uint32_t touch = 0;
-  auto touch_row = [&]() {
-    if (sg < a.n_seg) {
-      const FusedSeg& s = a.seg[sg];
-      const uint8_t* row = s.w + (size_t)i * s.row_bytes;
-      const size_t off = min((size_t)128 * lane, s.row_bytes - 4);
-      touch = *reinterpret_cast<const uint32_t*>((uintptr_t)(row + off) & ~(uintptr_t)3);
-    }
-  };
-  if constexpr (!NORM) touch_row();
-  // The residual an output row is added to is read now, under the rest.
-  float addv = 0.f;
-  if (sg < a.n_seg && a.seg[sg].add && lane == 0) addv = a.seg[sg].add[i];
-  const float* x = a.x;
+  float addv = 0.f;  // the residual an output row is added to
+  if (sg < a.n_seg) {
+    const FusedSeg& s = a.seg[sg];
+    const uint8_t* row = s.w + (size_t)i * s.row_bytes;
+    const size_t off = min((size_t)128 * lane, s.row_bytes - 4);
+    touch = *reinterpret_cast<const uint32_t*>((uintptr_t)(row + off) & ~(uintptr_t)3);
+    if (s.add && lane == 0) addv = s.add[i];
+  }
+  float inv = 1.f;
   if constexpr (NORM) {
-#pragma clang fp contract(off)
-    // The normalized row, x * inv * w left to right in f32 (norm.rs:55-57),
-    // staged in LDS for the quantizers. Each thread loads its values of x
-    // and w once (x <= 8192 values: at most 16 per thread), so the sum of
-    // squares and the scaling cost one memory round trip between them.
-    constexpr int NT = 64 * kFusedWaves, PER = kFusedMaxKBlocks * 256 / NT;
-    __shared__ float xs[kFusedMaxKBlocks * 256];
+    // norm.rs:55-57: x * inv * w left to right in f32.
     __shared__ double red[kFusedWaves];
-    const int n = a.nbk * 256;
-    float xr[PER], wr[PER];
-#pragma unroll
-    for (int r = 0; r < PER; ++r) {
-      const int j = threadIdx.x + r * NT;
-      xr[r] = j < n ? a.x[j] : 0.f;
-      wr[r] = j < n ? a.norm_w[j] : 0.f;
-    }
-    asm volatile("" ::: "memory");  // the row loads above issue first
-    touch_row();
     double ss = 0.0;
 #pragma unroll
-    for (int r = 0; r < PER; ++r) ss += (double)xr[r] * (double)xr[r];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    for (int r = 0; r < 4 * NB; ++r) {
+      const double v = (int)threadIdx.x + 64 * kFusedWaves * r < n ? (double)xs[r] : 0.0;
+      ss += v * v;
+    }
+    ss = wave_sum_tree_f64(ss);
     if (lane == 0) red[wave] = ss;
     __syncthreads();
     double tot = 0.0;
 #pragma unroll
     for (int w = 0; w < kFusedWaves; ++w) tot += red[w];
-    const float inv = (float)(1.0 / sqrt(tot / (double)n + (double)a.eps));
-#pragma unroll
-    for (int r = 0; r < PER; ++r) {
-      const int j = threadIdx.x + r * NT;
-      if (j < n) xs[j] = xr[r] * inv * wr[r];
-    }
-    __syncthreads();
-    x = xs;
+    inv = (float)(1.0 / sqrt(tot / (double)n + (double)a.eps));
   }
-  if (need_k)
-    for (int b = wave; b < a.nbk; b += kFusedWaves) quantize_block_q8_k(x + (size_t)b * 256, &lk[b], lane);
-  if (need_0)
-    for (int b = 2 * wave + (lane >> 5); b < a.nb0; b += 2 * kFusedWaves)
-      quantize_block_q8_0(x + (size_t)b * 32, &l0[b], lane & 31);
+#pragma unroll
+  for (int u = 0; u < NB; ++u) {
+    const int b = wave + kFusedWaves * u;
+    if (b >= a.nbk) break;  // wave-uniform
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = NORM ? xv[u][e] * inv * wv[u][e] : xv[u][e];
+    if (need_k) store_q8_k(quantize_lane_q8_k(v), &lk[b], lane);
+    if (need_0) {
+      const Q80Lane z = quantize_lane_q8_0(v);
+      rv_block_q8_0* blk = &l0[8 * b + (lane >> 3)];
+      *reinterpret_cast<uint32_t*>(blk->qs + 4 * (lane & 7)) = z.q;
+      if ((lane & 7) == 0) blk->d = z.d;
+    }
+  }
   __syncthreads();
   asm volatile("" ::"v"(touch));
   if (sg >= a.n_seg) return;  // wave-uniform
@@ -643,11 +663,21 @@ HipStatus launch_fused_proj(const FusedProjArgs& a, hipStream_t s) {
   long rows = 0;
   for (int i = 0; i < a.n_seg; ++i) rows += a.n_rows[i];
   if (rows == 0) return st;
-  const dim3 grid((unsigned)((rows + kFusedWaves - 1) / kFusedWaves));
-  if (a.norm_w)
-    hipLaunchKernelGGL(fused_proj_kernel<true>, grid, dim3(64 * kFusedWaves), 0, s, a);
-  else
-    hipLaunchKernelGGL(fused_proj_kernel<false>, grid, dim3(64 * kFusedWaves), 0, s, a);
+  const dim3 grid((unsigned)((rows + kFusedWaves - 1) / kFusedWaves)), block(64 * kFusedWaves);
+#define RV_FUSED(NB)                                                          \
+  if (a.norm_w)                                                               \
+    hipLaunchKernelGGL((fused_proj_kernel<true, NB>), grid, block, 0, s, a);  \
+  else                                                                        \
+    hipLaunchKernelGGL((fused_proj_kernel<false, NB>), grid, block, 0, s, a)
+  if (a.nbk <= kFusedWaves) {
+    RV_FUSED(1);
+  } else if (a.nbk <= 2 * kFusedWaves) {
+    RV_FUSED(2);
+  } else {
+    RV_FUSED(4);
+  }
+#undef RV_FUSED
+  static_assert(kFusedMaxKBlocks == 4 * kFusedWaves, "the widest row");
   st.e = hipGetLastError();
   if (st.e != hipSuccess) st.what = "fused projection launch";
   return st;
