@@ -29,32 +29,34 @@ __device__ __forceinline__ float f16_bits_to_f32(uint32_t bits) {
   return (float)__builtin_bit_cast(_Float16, (uint16_t)(bits & 0xFFFFu));
 }
 
-// 32 bytes at a 2-byte-aligned address, as 8 little-endian dwords, reading
-// nothing outside [a, a + 32) except the two bytes before `a` (which the
-// callers' layouts guarantee belong to the same block).
-__device__ __forceinline__ void load32_a2(const uint8_t* a, uint32_t (&w)[8]) {
-  if (((uintptr_t)a & 2) == 0) {
-    const uint32_t* p = reinterpret_cast<const uint32_t*>(a);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) w[k] = p[k];
-    return;
-  }
-  const uint32_t* p = reinterpret_cast<const uint32_t*>(a - 2);  // bytes a-2 .. a+1
+// 32 bytes at a 2-byte-aligned address as raw dwords: aligned-down reads plus
+// a 2-byte tail, reading nothing outside [a, a + 32) except the two bytes
+// before `a` (which the callers' layouts guarantee belong to the same block).
+// fix32 realigns them, so the loads can be issued ahead of their use.
+struct Raw32 {
   uint32_t e[8];
+  uint32_t tail, odd;
+};
+__device__ __forceinline__ Raw32 raw32_a2(const uint8_t* a) {
+  Raw32 r;
+  r.odd = (uint32_t)(uintptr_t)a & 2;
+  const uint32_t* p = reinterpret_cast<const uint32_t*>(a - r.odd);
 #pragma unroll
-  for (int k = 0; k < 7; ++k) e[k + 1] = p[k + 1];  // bytes a+2+4k .. a+5+4k
-  e[0] = p[0];
-  const uint32_t tail = *reinterpret_cast<const uint16_t*>(a + 30);
+  for (int k = 0; k < 8; ++k) r.e[k] = p[k];
+  r.tail = *reinterpret_cast<const uint16_t*>(a + 30);
+  return r;
+}
+__device__ __forceinline__ void fix32(const Raw32& r, uint32_t (&w)[8]) {
 #pragma unroll
-  for (int k = 0; k < 7; ++k) w[k] = __builtin_amdgcn_alignbyte(e[k + 1], e[k], 2);
-  w[7] = (e[7] >> 16) | (tail << 16);
+  for (int k = 0; k < 7; ++k) w[k] = __builtin_amdgcn_alignbyte(r.e[k + 1], r.e[k], r.odd);
+  w[7] = r.odd ? (r.e[7] >> 16) | (r.tail << 16) : r.e[7];
 }
 
 // Sum over the 8 lanes of an aligned lane group (exact for integers).
 __device__ __forceinline__ int sum8_lanes(int v) {
-  v += __shfl_xor(v, 1, 64);
-  v += __shfl_xor(v, 2, 64);
-  v += __shfl_xor(v, 4, 64);
+  v += __builtin_amdgcn_update_dpp(0, v, DPP_QUAD_XOR1, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, DPP_QUAD_XOR2, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, DPP_ROW_HALF_MIRROR, 0xF, 0xF, false);
   return v;
 }
 
@@ -103,126 +105,175 @@ __device__ __forceinline__ ActK act_from_block(const rv_block_q8_k* __restrict__
   return r;
 }
 
+// What a lane loads of its weight block: k-quants, lane j of the block's 8;
+// Q8_0, the whole 32-weight block.
+template <int FMT>
+struct BlockRaw;
+template <>
+struct BlockRaw<RV_QF_Q4_K> {
+  u32x4a hdr, q[2];
+};
+template <>
+struct BlockRaw<RV_QF_Q5_K> {
+  u32x4a hdr, q[2], h[2];
+};
+template <>
+struct BlockRaw<RV_QF_Q6_K> {
+  Raw32 ql, qh;
+  uint32_t sc, d;
+};
+template <>
+struct BlockRaw<RV_QF_Q8_0> {
+  Raw32 q;
+  uint32_t d;
+};
+
+template <int FMT>
+__device__ __forceinline__ void load_block(BlockRaw<FMT>& w, const uint8_t* __restrict__ blk, int j) {
+  if constexpr (FMT == RV_QF_Q8_0) {
+    w.d = *reinterpret_cast<const uint16_t*>(blk);
+    w.q = raw32_a2(blk + 2);
+  } else if constexpr (FMT == RV_QF_Q6_K) {
+    const int half = j >> 2, grp = j & 3;
+    w.ql = raw32_a2(blk + 64 * half + 32 * (grp & 1));
+    w.qh = raw32_a2(blk + 128 + 32 * half);
+    w.sc = *reinterpret_cast<const uint16_t*>(blk + 192 + 2 * j);
+    w.d = *reinterpret_cast<const uint16_t*>(blk + 208);
+  } else {
+    constexpr bool kQ5 = FMT == RV_QF_Q5_K;
+    w.hdr = *reinterpret_cast<const u32x4a*>(blk);
+    const u32x4a* qp = reinterpret_cast<const u32x4a*>(blk + (kQ5 ? 48 : 16) + 32 * (j >> 1));
+    w.q[0] = qp[0], w.q[1] = qp[1];
+    if constexpr (kQ5) {
+      const u32x4a* hp = reinterpret_cast<const u32x4a*>(blk + 16);
+      w.h[0] = hp[0], w.h[1] = hp[1];
+    }
+  }
+}
+
 // One super-block's float contribution for the k-quants, computed by the 8
 // lanes of a group, lane j owning sub-block j (Q4_K/Q5_K: 32 weights) or
 // the two 16-weight sub-blocks 2j, 2j+1 (Q6_K); every lane of the group
 // returns the same value.
+//  - Q4_K / Q5_K: k_quant_affine_block with the expansions (dot.rs:56-143):
+//    d*sumi - dmin*sumi_mins, d = f16(d)*y.d, dmin = f16(dmin)*y.d.
+//  - Q6_K: vec_dot_q6_k_q8_k (dot.rs:150-179): lane j = 4 half + group holds
+//    weights 32j .. 32j+31: ql nibbles (byte l + 32 (group & 1) of the half,
+//    high nibble for groups 2, 3) and two qh bits (2 group). The stored values
+//    are q + 32 in 0..63; sum (q+32)a - 32 sum a, with sum a the activation
+//    bsums.
 template <int FMT>
-__device__ __forceinline__ float kq_block(const uint8_t* __restrict__ blk, const ActK& y, int j);
+__device__ __forceinline__ float kq_block(const BlockRaw<FMT>& w, const ActK& y, int j) {
+#pragma clang fp contract(off)
+  if constexpr (FMT == RV_QF_Q6_K) {
+    const int grp = j & 3;
+    uint32_t ql[8], qh[8];
+    fix32(w.ql, ql);
+    fix32(w.qh, qh);
+    int lo = 0, hi = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t nib = (grp >> 1) ? (ql[k] >> 4) & 0x0F0F0F0Fu : ql[k] & 0x0F0F0F0Fu;
+      const uint32_t v = nib | (((qh[k] >> (2 * grp)) & 0x03030303u) << 4);
+      if (k < 4)
+        lo = dot4(v, y.a[k], lo);
+      else
+        hi = dot4(v, y.a[k], hi);
+    }
+    lo -= 32 * y.bs_lo;
+    hi -= 32 * y.bs_hi;
+    const int sc_lo = (int)(int8_t)(w.sc & 0xFF), sc_hi = (int)(int8_t)(w.sc >> 8);
+    const int sumi = sum8_lanes(sc_lo * lo + sc_hi * hi);
+    const float d = f16_bits_to_f32(w.d);
+    return d * y.d * (float)sumi;
+  } else {
+    const uint32_t s[3] = {w.hdr[1], w.hdr[2], w.hdr[3]};
+    int acc = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      uint32_t v = (w.q[k >> 2][k & 3] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+      if constexpr (FMT == RV_QF_Q5_K) v |= ((w.h[k >> 2][k & 3] >> j) & 0x01010101u) << 4;
+      acc = dot4(v, y.a[k], acc);
+    }
+    int sc, m;
+    scale_min_k4(j, s, sc, m);
+    const int sumi = sum8_lanes(sc * acc);
+    const int sumi_mins = sum8_lanes(m * (y.bs_lo + y.bs_hi));
+    const float d = f16_bits_to_f32(w.hdr[0]) * y.d;
+    const float dmin = f16_bits_to_f32(w.hdr[0] >> 16) * y.d;
+    return d * (float)sumi - dmin * (float)sumi_mins;
+  }
+}
 
-// k_quant_affine_block with the q4_K / q5_K expansions (dot.rs:56-143):
-// d*sumi - dmin*sumi_mins, d = f16(d)*y.d, dmin = f16(dmin)*y.d.
+// One row against its activation blocks (global memory or LDS), every lane
+// returning the row's sum, added in block order. k-quants: 8 super-blocks per
+// pass (lane group b); Q8_0 (vec_dot_q8_0_q8_0, dot.rs:185-201): lane per
+// 32-weight block, 64 per pass, sumf += sumi * (f16(d) * y.d). The first P
+// passes' weights come in `pre` (row_prefetch), loaded ahead.
 template <int FMT>
-__device__ __forceinline__ float affine_block(const uint8_t* __restrict__ blk, const ActK& y, int j) {
-#pragma clang fp contract(off)
-  constexpr bool kQ5 = FMT == RV_QF_Q5_K;
-  const uint32_t dd = *reinterpret_cast<const uint32_t*>(blk);
-  const uint32_t* sp = reinterpret_cast<const uint32_t*>(blk + 4);
-  const uint32_t s[3] = {sp[0], sp[1], sp[2]};
-  const u32x4a* qp = reinterpret_cast<const u32x4a*>(blk + (kQ5 ? 48 : 16) + 32 * (j >> 1));
-  const u32x4a q0 = qp[0], q1 = qp[1];
-  const uint32_t q[8] = {q0[0], q0[1], q0[2], q0[3], q1[0], q1[1], q1[2], q1[3]};
-  uint32_t qh[8];
-  if constexpr (kQ5) {
-    const u32x4a* hp = reinterpret_cast<const u32x4a*>(blk + 16);
-    const u32x4a h0 = hp[0], h1 = hp[1];
-    qh[0] = h0[0], qh[1] = h0[1], qh[2] = h0[2], qh[3] = h0[3];
-    qh[4] = h1[0], qh[5] = h1[1], qh[6] = h1[2], qh[7] = h1[3];
-  }
-  int acc = 0;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    uint32_t w = (j & 1) ? (q[k] >> 4) & 0x0F0F0F0Fu : q[k] & 0x0F0F0F0Fu;
-    if constexpr (kQ5) w |= ((qh[k] >> j) & 0x01010101u) << 4;
-    acc = dot4(w, y.a[k], acc);
-  }
-  int sc, m;
-  scale_min_k4(j, s, sc, m);
-  const int sumi = sum8_lanes(sc * acc);
-  const int sumi_mins = sum8_lanes(m * (y.bs_lo + y.bs_hi));
-  const float d = f16_bits_to_f32(dd) * y.d;
-  const float dmin = f16_bits_to_f32(dd >> 16) * y.d;
-  return d * (float)sumi - dmin * (float)sumi_mins;
-}
-
-template <>
-__device__ __forceinline__ float kq_block<RV_QF_Q4_K>(const uint8_t* blk, const ActK& y, int j) {
-  return affine_block<RV_QF_Q4_K>(blk, y, j);
-}
-template <>
-__device__ __forceinline__ float kq_block<RV_QF_Q5_K>(const uint8_t* blk, const ActK& y, int j) {
-  return affine_block<RV_QF_Q5_K>(blk, y, j);
-}
-
-// vec_dot_q6_k_q8_k (dot.rs:150-179): lane j = 4 half + group holds weights
-// 32j .. 32j+31: ql nibbles (byte l + 32 (group & 1) of the half, high
-// nibble for groups 2, 3) and two qh bits (2 group). The stored values are
-// q + 32 in 0..63; sum (q+32)a - 32 sum a, with sum a the activation bsums.
-template <>
-__device__ __forceinline__ float kq_block<RV_QF_Q6_K>(const uint8_t* blk, const ActK& y, int j) {
-#pragma clang fp contract(off)
-  const int half = j >> 2, grp = j & 3;
-  uint32_t ql[8], qh[8];
-  load32_a2(blk + 64 * half + 32 * (grp & 1), ql);
-  load32_a2(blk + 128 + 32 * half, qh);
-  int lo = 0, hi = 0;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const uint32_t nib = (grp >> 1) ? (ql[k] >> 4) & 0x0F0F0F0Fu : ql[k] & 0x0F0F0F0Fu;
-    const uint32_t w = nib | (((qh[k] >> (2 * grp)) & 0x03030303u) << 4);
-    if (k < 4)
-      lo = dot4(w, y.a[k], lo);
-    else
-      hi = dot4(w, y.a[k], hi);
-  }
-  lo -= 32 * y.bs_lo;
-  hi -= 32 * y.bs_hi;
-  const uint32_t scp = *reinterpret_cast<const uint16_t*>(blk + 192 + 2 * j);
-  const int sc_lo = (int)(int8_t)(scp & 0xFF), sc_hi = (int)(int8_t)(scp >> 8);
-  const int sumi = sum8_lanes(sc_lo * lo + sc_hi * hi);
-  const float d = f16_bits_to_f32(*reinterpret_cast<const uint16_t*>(blk + 208));
-  return d * y.d * (float)sumi;
-}
-
-// One k-quant row against its Q8_K activation blocks (global memory or
-// LDS), every lane returning the row's sum: 8 super-blocks per pass (lane
-// group b), added in block order.
+constexpr int kPassBlocks = FMT == RV_QF_Q8_0 ? 64 : 8;
 template <int FMT>
-__device__ __forceinline__ float kq_row(const uint8_t* __restrict__ row, int nb, const rv_block_q8_k* __restrict__ acts,
-                                        int lane) {
-  constexpr int BB = FMT == RV_QF_Q4_K ? 144 : FMT == RV_QF_Q5_K ? 176 : 210;
-  const int bl = lane >> 3, j = lane & 7;
-  float sumf = 0.f;
-  for (int b0 = 0; b0 < nb; b0 += 8) {
-    const int b = min(b0 + bl, nb - 1);  // groups past the row recompute its last block (unused)
-    const float c = kq_block<FMT>(row + (size_t)b * BB, act_from_block(acts + b, j), j);
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (b0 + k < nb) sumf += lane_f(c, 8 * k);
-  }
-  return sumf;
+constexpr int kBlockBytes = FMT == RV_QF_Q4_K ? 144 : FMT == RV_QF_Q5_K ? 176 : FMT == RV_QF_Q6_K ? 210 : 34;
+
+template <int FMT>
+__device__ __forceinline__ void load_pass(BlockRaw<FMT>& w, const uint8_t* __restrict__ row, int nb, int b0, int lane) {
+  // Groups past the row re-read its last block (unused).
+  const int b = min(b0 + (FMT == RV_QF_Q8_0 ? lane : lane >> 3), nb - 1);
+  load_block<FMT>(w, row + (size_t)b * kBlockBytes<FMT>, lane & 7);
 }
 
-// vec_dot_q8_0_q8_0 (dot.rs:185-201): lane per 32-weight block, 64 blocks
-// per pass, sumf += sumi * (f16(d) * y.d) in block order.
-__device__ __forceinline__ float q80_row(const uint8_t* __restrict__ row, int nb, const rv_block_q8_0* __restrict__ acts,
-                                         int lane) {
+template <int FMT>
+__device__ __forceinline__ float pass_value(const BlockRaw<FMT>& w, int nb, int b0, const void* __restrict__ acts,
+                                            int lane) {
 #pragma clang fp contract(off)
-  float sumf = 0.f;
-  for (int b0 = 0; b0 < nb; b0 += 64) {
-    const int b = min(b0 + lane, nb - 1);
-    const uint8_t* blk = row + (size_t)b * 34;
-    uint32_t w[8];
-    load32_a2(blk + 2, w);
-    const int* a = reinterpret_cast<const int*>(acts[b].qs);
+  if constexpr (FMT == RV_QF_Q8_0) {
+    const rv_block_q8_0* y = reinterpret_cast<const rv_block_q8_0*>(acts) + min(b0 + lane, nb - 1);
+    uint32_t q[8];
+    fix32(w.q, q);
+    const int* a = reinterpret_cast<const int*>(y->qs);
     int s = 0;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) s = dot4(w[k], a[k], s);
-    const float c = (float)s * (f16_bits_to_f32(*reinterpret_cast<const uint16_t*>(blk)) * acts[b].d);
-    const int n = min(64, nb - b0);
-    for (int k = 0; k < n; ++k) sumf += lane_f(c, k);
+    for (int k = 0; k < 8; ++k) s = dot4(q[k], a[k], s);
+    return (float)s * (f16_bits_to_f32(w.d) * y->d);
+  } else {
+    const rv_block_q8_k* y = reinterpret_cast<const rv_block_q8_k*>(acts) + min(b0 + (lane >> 3), nb - 1);
+    return kq_block<FMT>(w, act_from_block(y, lane & 7), lane & 7);
+  }
+}
+
+template <int FMT>
+__device__ __forceinline__ float add_pass(float sumf, float c, int nb, int b0) {
+  constexpr int N = kPassBlocks<FMT>, S = 64 / N;
+  if (b0 + N <= nb) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) sumf += lane_f(c, S * k);
+  } else {
+    for (int k = 0; k < nb - b0; ++k) sumf += lane_f(c, S * k);
   }
   return sumf;
+}
+
+template <int FMT, int P>
+__device__ __forceinline__ float row_sum(const BlockRaw<FMT> (&pre)[P], const uint8_t* __restrict__ row, int nb,
+                                         const void* __restrict__ acts, int lane) {
+  constexpr int N = kPassBlocks<FMT>;
+  float sumf = 0.f;
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+    if (N * p < nb) sumf = add_pass<FMT>(sumf, pass_value<FMT>(pre[p], nb, N * p, acts, lane), nb, N * p);
+  for (int b0 = N * P; b0 < nb; b0 += N) {
+    BlockRaw<FMT> w;
+    load_pass<FMT>(w, row, nb, b0, lane);
+    sumf = add_pass<FMT>(sumf, pass_value<FMT>(w, nb, b0, acts, lane), nb, b0);
+  }
+  return sumf;
+}
+
+template <int FMT, int P>
+__device__ __forceinline__ void row_prefetch(BlockRaw<FMT> (&pre)[P], const uint8_t* __restrict__ row, int nb,
+                                             int lane) {
+#pragma unroll
+  for (int p = 0; p < P; ++p) load_pass<FMT>(pre[p], row, nb, kPassBlocks<FMT> * p, lane);
 }
 
 // quantize_row_q8_k (quantize.rs:71-106) of one block by one wave, lane l
@@ -343,15 +394,6 @@ __global__ __launch_bounds__(256) void quantize_both_kernel(const float* __restr
   }
 }
 
-__device__ __forceinline__ float row_dot(uint32_t fmt, const uint8_t* row, int nb, const void* acts, int lane) {
-  switch (fmt) {
-    case RV_QF_Q4_K: return kq_row<RV_QF_Q4_K>(row, nb, (const rv_block_q8_k*)acts, lane);
-    case RV_QF_Q5_K: return kq_row<RV_QF_Q5_K>(row, nb, (const rv_block_q8_k*)acts, lane);
-    case RV_QF_Q6_K: return kq_row<RV_QF_Q6_K>(row, nb, (const rv_block_q8_k*)acts, lane);
-    default: return q80_row(row, nb, (const rv_block_q8_0*)acts, lane);
-  }
-}
-
 constexpr int kRowsPerWG = 4;
 
 // out[i] = row(row_lo + i) . acts for i < n_rows, acts quantized blocks in
@@ -364,11 +406,9 @@ __global__ __launch_bounds__(64 * kRowsPerWG) void gemv_rows_kernel(const uint8_
   const int i = (int)blockIdx.x * kRowsPerWG + (threadIdx.x >> 6);
   if (i >= n_rows) return;  // wave-uniform
   const uint8_t* row = w + (size_t)(row_lo + i) * row_bytes;
-  float v;
-  if constexpr (FMT == RV_QF_Q8_0)
-    v = q80_row(row, nb, (const rv_block_q8_0*)acts, lane);
-  else
-    v = kq_row<FMT>(row, nb, (const rv_block_q8_k*)acts, lane);
+  BlockRaw<FMT> pre[1];
+  row_prefetch<FMT, 1>(pre, row, nb, lane);
+  const float v = row_sum<FMT, 1>(pre, row, nb, acts, lane);
   if (lane == 0) out[i] = v;
 }
 
@@ -411,24 +451,23 @@ __device__ __forceinline__ double wave_sum_tree_f64(double x) {
   return x;
 }
 
-// NB: Q8_K blocks per wave (x holds at most 256 * kFusedWaves * NB values).
-template <bool NORM, int NB>
-__global__ __launch_bounds__(64 * kFusedWaves) void fused_proj_kernel(FusedProjArgs a) {
+// One wave's part of a fused projection: its weight row (FMT) is loaded while
+// the workgroup (normalizes and) quantizes x; NB Q8_K blocks of x per wave.
+// Every wave of the workgroup comes through here, each with its row's FMT, and
+// passes the same barriers; a wave past the last row has live false.
+template <int FMT, bool NORM, int NB>
+__device__ __forceinline__ void fused_wave(const FusedProjArgs& a, const FusedSeg& s, int i, bool live, bool need_k,
+                                           bool need_0, int wave, int lane, rv_block_q8_k* lk, rv_block_q8_0* l0,
+                                           double* red) {
 #pragma clang fp contract(off)
   typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
-  __shared__ rv_block_q8_k lk[kFusedWaves * NB];
-  __shared__ rv_block_q8_0 l0[kFusedWaves * NB * 8];
-  // The wave index as a scalar: the row, its segment and the segment's
-  // fields are then wave-uniform, read with scalar loads from the kernel
-  // arguments (indexed from a vector register, each was a vector load of
-  // the argument segment that every later load waited behind).
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (a.gate_pos && *a.gate_pos > a.gate_max) return;  // the whole grid: its decode step was refused
-  const int first = (int)blockIdx.x * kFusedWaves;
+  constexpr int P = FMT != RV_QF_Q8_0 && NB > 1 ? 2 : 1;  // passes whose weights are loaded ahead
+  const int nbw = FMT == RV_QF_Q8_0 ? a.nb0 : a.nbk;
   // The lane's four values of each of the wave's blocks (blocks past the row
   // re-read its last), straight into the quantizers' registers; with the norm
   // also its weight and, for the sum of squares, the values in the summing
-  // order (thread t: t, t + 512, ..).
+  // order (thread t: t, t + 512, ..). They are issued ahead of the weights,
+  // since loads retire in order.
   f32x4a xv[NB], wv[NB];
   float xs[NORM ? 4 * NB : 1];
   const int n = a.nbk * 256;
@@ -437,42 +476,22 @@ __global__ __launch_bounds__(64 * kFusedWaves) void fused_proj_kernel(FusedProjA
     for (int r = 0; r < 4 * NB; ++r) xs[r] = a.x[min((int)threadIdx.x + 64 * kFusedWaves * r, n - 1)];
   }
 #pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    const int at = 256 * min(wave + kFusedWaves * i, a.nbk - 1) + 4 * lane;
-    xv[i] = *reinterpret_cast<const f32x4a*>(a.x + at);
-    if constexpr (NORM) wv[i] = *reinterpret_cast<const f32x4a*>(a.norm_w + at);
+  for (int u = 0; u < NB; ++u) {
+    const int at = 256 * min(wave + kFusedWaves * u, a.nbk - 1) + 4 * lane;
+    xv[u] = *reinterpret_cast<const f32x4a*>(a.x + at);
+    if constexpr (NORM) wv[u] = *reinterpret_cast<const f32x4a*>(a.norm_w + at);
   }
-  asm volatile("" ::: "memory");  // the row loads above issue first
-  // The segments this workgroup's rows touch decide which forms it needs.
-  bool need_k = false, need_0 = false;
-  {
-    int lo = 0;
-    for (int sg = 0; sg < a.n_seg; ++sg) {
-      const int hi = lo + a.n_rows[sg];
-      if (first < hi && first + kFusedWaves > lo) (a.seg[sg].fmt == RV_QF_Q8_0 ? need_0 : need_k) = true;
-      lo = hi;
-    }
-  }
-  int i = first + wave, sg = 0;
-  while (sg < a.n_seg && i >= a.n_rows[sg]) i -= a.n_rows[sg++];
-  // This wave's weight row starts streaming while the workgroup quantizes:
-  // one dword from each of its 128-byte lines (lane l: byte 128 l, clamped
-  // to the row and aligned down; the matrix base is 4-byte aligned, so the
-  // address stays inside it). The value is consumed only after the barrier,
-  // so nothing waits for it.
-  uint32_t touch = 0;
-  float addv = 0.f;  // the residual an output row is added to
-  if (sg < a.n_seg) {
-    const FusedSeg& s = a.seg[sg];
-    const uint8_t* row = s.w + (size_t)i * s.row_bytes;
-    const size_t off = min((size_t)128 * lane, s.row_bytes - 4);
-    touch = *reinterpret_cast<const uint32_t*>((uintptr_t)(row + off) & ~(uintptr_t)3);
-    if (s.add && lane == 0) addv = s.add[i];
-  }
+  asm volatile("" ::: "memory");
+  const uint8_t* row = s.w + (size_t)i * s.row_bytes;
+  BlockRaw<FMT> pre[P];
+  row_prefetch<FMT, P>(pre, row, nbw, lane);
+  float addv = 0.f;  // the residual the output row is added to
+  if (s.add && lane == 0) addv = s.add[i];
+  const uint32_t gate = a.gate_pos ? *a.gate_pos : 0u;
+  asm volatile("" ::: "memory");  // issued before the barriers
   float inv = 1.f;
   if constexpr (NORM) {
     // norm.rs:55-57: x * inv * w left to right in f32.
-    __shared__ double red[kFusedWaves];
     double ss = 0.0;
 #pragma unroll
     for (int r = 0; r < 4 * NB; ++r) {
@@ -503,13 +522,48 @@ __global__ __launch_bounds__(64 * kFusedWaves) void fused_proj_kernel(FusedProjA
     }
   }
   __syncthreads();
-  asm volatile("" ::"v"(touch));
-  if (sg >= a.n_seg) return;  // wave-uniform
-  const FusedSeg& s = a.seg[sg];
-  const bool q80 = s.fmt == RV_QF_Q8_0;
-  const float v = row_dot(s.fmt, s.w + (size_t)i * s.row_bytes, q80 ? a.nb0 : a.nbk,
-                          q80 ? (const void*)l0 : (const void*)lk, lane);
+  if (!live || gate > a.gate_max) return;  // (the whole grid's decode step was refused: nothing is written)
+  const float v = row_sum<FMT, P>(pre, row, nbw, FMT == RV_QF_Q8_0 ? (const void*)l0 : (const void*)lk, lane);
   if (lane == 0) s.out[i] = s.add ? addv + v : v;
+}
+
+// NB: Q8_K blocks per wave (x holds at most 256 * kFusedWaves * NB values).
+template <bool NORM, int NB>
+__global__ __launch_bounds__(64 * kFusedWaves) void fused_proj_kernel(FusedProjArgs a) {
+  __shared__ rv_block_q8_k lk[kFusedWaves * NB];
+  __shared__ rv_block_q8_0 l0[kFusedWaves * NB * 8];
+  __shared__ double red[kFusedWaves];
+  // The wave index as a scalar: the row, its segment and the segment's
+  // fields are then wave-uniform, read with scalar loads from the kernel
+  // arguments (indexed from a vector register, each was a vector load of
+  // the argument segment that every later load waited behind).
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int first = (int)blockIdx.x * kFusedWaves;
+  // The segments this workgroup's rows touch decide which forms it needs.
+  bool need_k = false, need_0 = false;
+  {
+    int lo = 0;
+    for (int sg = 0; sg < a.n_seg; ++sg) {
+      const int hi = lo + a.n_rows[sg];
+      if (first < hi && first + kFusedWaves > lo) (a.seg[sg].fmt == RV_QF_Q8_0 ? need_0 : need_k) = true;
+      lo = hi;
+    }
+  }
+  int i = first + wave, sg = 0;
+  while (sg < a.n_seg && i >= a.n_rows[sg]) i -= a.n_rows[sg++];
+  const bool live = sg < a.n_seg;
+  if (!live) {  // past the last row: quantizes beside the others, on the last segment that has rows
+    sg = a.n_seg - 1;
+    while (a.n_rows[sg] == 0) --sg;
+    i = a.n_rows[sg] - 1;
+  }
+  const FusedSeg& s = a.seg[sg];
+  switch (s.fmt) {
+    case RV_QF_Q4_K: return fused_wave<RV_QF_Q4_K, NORM, NB>(a, s, i, live, need_k, need_0, wave, lane, lk, l0, red);
+    case RV_QF_Q5_K: return fused_wave<RV_QF_Q5_K, NORM, NB>(a, s, i, live, need_k, need_0, wave, lane, lk, l0, red);
+    case RV_QF_Q6_K: return fused_wave<RV_QF_Q6_K, NORM, NB>(a, s, i, live, need_k, need_0, wave, lane, lk, l0, red);
+    default: return fused_wave<RV_QF_Q8_0, NORM, NB>(a, s, i, live, need_k, need_0, wave, lane, lk, l0, red);
+  }
 }
 
 __global__ __launch_bounds__(1024) void rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w,

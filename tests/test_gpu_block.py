@@ -113,6 +113,16 @@ def test_attn_block_matches_the_oracle_composition(elem):
                0xB10C)
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hidden", [(2, 1, 256), (8, 1, 2304), (36, 4, 4352)])
+def test_attn_block_at_the_edges_of_blocks_per_wave(n_heads, n_kv, hidden):
+    # Rows of 1, 9 and 17 activation blocks in (the norm form) and of 1, 4 and
+    # 18 out: one, two and four blocks per wave, with a partial last one.
+    torch = torch_cuda()
+    Q = oracle
+    run_tokens(torch, f"hidden {hidden}", n_heads, n_kv, hidden, (Q.RV_QF_Q6_K, Q.RV_QF_Q5_K, Q.RV_QF_Q4_K), "f32", 33,
+               2, 0xB1A0 + hidden)
+
+
 def test_attn_block_other_formats_and_geometry():
     # v as Q4_K and o as Q6_K (both appear in the v0 model), 16 q heads over 2 kv heads.
     torch = torch_cuda()
