@@ -299,7 +299,8 @@ struct Chunk<_Float16> {
 //     exp is computed once;
 //   O^T[d][m] += sum_t V[t][d] P^T[t][m]: 8 x 4 MFMAs; the accumulator layout
 //     of S^T is exactly the B layout P^T needs (step r takes rows 4k + r), and
-//     lane (i, k) holds V[4k + r][8i .. 8i+7], so output block b is d = 8i + b.
+//     lane (i, k) holds eight columns of V[4k + r], one per output block (fp32
+//     4i .. + 3 and 64 + 4i .. + 3, f16 8i .. + 7).
 // Each wave keeps D tiles in flight in a register ring (D = 1 when the grid
 // holds two waves per SIMD):
 // the first D tiles' loads are issued before anything waits, and the loads
@@ -528,33 +529,77 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
       __syncthreads();
     }
   }
+  // A global load whose neighbouring lanes fall into different rows costs the
+  // CU's address unit 64 cycles, one over consecutive lanes 16; the MFMA
+  // operands of q and K have a row per lane. So the wave loads both in row
+  // order and turns them around through its own part of the LDS (the bytes of
+  // its merge rows; a wave's LDS operations run in order, so no barrier), with
+  // a row's 16-byte chunks permuted by the row: 16 rows' writes and reads of
+  // one chunk fall on all banks. Against loads in operand order (per call,
+  // one layer's graph, L2-resident up to 4096): f16 32768 positions 19.5 ->
+  // 17.8 us, 2000 7.06 -> 6.89; fp32 16384 19.7 -> 17.8, 2000 8.35 -> 7.95, 400
+  // 7.06 -> 6.60; fp32 4096 the same; up to 100 positions +0.1-0.3 us where the
+  // rows are in the L2 (the turn-around's latency) and -0.1 where they are not.
+  char* const turn = lds_raw + (size_t)wave * (16 * (kD + 4) * (int)sizeof(float));
   float qv[32];
+  // Row li of q: head li of the group (the first past it, unused). Loads of
+  // 16 bytes at q's 4-byte alignment; two heads per load.
+  typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
+  f32x4a qr[8];
   {
-    // q may be only 4-byte aligned: scalar loads (once per workgroup). (Staging
-    // the group's rows through LDS with coalesced loads measured slower: its
-    // barrier costs more than the gather.)
-    const float* qp = q + (size_t)(kvh * group + (col_ok ? li : 0)) * kD;
+    const float* qp = q + (size_t)(kvh * group) * kD + 4 * (lane & 31);
 #pragma unroll
-    for (int c = 0; c < NKC; ++c)
-#pragma unroll
-      for (int e = 0; e < E; ++e) qv[c * E + e] = qp[E * (lk + 4 * c) + e];
+    for (int i = 0; i < 8; ++i)
+      if (2 * i < group) qr[i] = *reinterpret_cast<const f32x4a*>(qp + (size_t)min(2 * i + (lane >> 5), group - 1) * kD);
   }
+  auto turn_q = [&]() {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (2 * i < group) {
+        const int h = 2 * i + (lane >> 5);
+        *reinterpret_cast<f32x4*>(turn + 512 * h + 16 * ((lane & 31) ^ h)) = qr[i];
+      }
+    const int h = col_ok ? li : 0;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {  // chunk of four: E = 4 takes lk + 4 c, E = 8 two of 2 (lk + 4 (c / 2))
+      const int k = E == 4 ? lk + 4 * c : 2 * (lk + 4 * (c >> 1)) + (c & 1);
+      const f32x4 v = *reinterpret_cast<const f32x4*>(turn + 512 * h + 16 * (k ^ h));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qv[4 * c + e] = v[e];
+    }
+  };
   // Rows past the split re-read its last row (in bounds, branch-free); their
   // scores are masked below, and tiles past the wave's share are loaded that
   // way but never computed. K and V are read once per call: non-temporal
-  // loads (config 2: 0.13 µs per call faster than plain loads).
+  // loads (config 2: 0.13 µs per call faster than plain loads). Chunk c of kb
+  // holds rows RC c + lane / CR, 16-byte chunk lane % CR of the row (turn_k
+  // makes it chunk lk + 4 c of row li).
+  constexpr int CR = kRowB / 16, RC = 64 / CR;
+  // V: lane li holds eight columns of its rows: fp32 4 li .. + 3 and 64 + 4 li
+  // .. + 3, so both loads are consecutive over the lanes; f16 8 li .. + 7.
   auto load_tile = [&](int j, CT (&kb)[NKC], CT (&vb)[NVC]) {
     const int t0 = t_begin + (wave + j * W) * 16;
-    const T* kp = kl + (size_t)min(t0 + li, t_end - 1) * kv_dim + col + E * lk;
 #pragma unroll
-    for (int c = 0; c < NKC; ++c) kb[c] = __builtin_nontemporal_load(reinterpret_cast<const CT*>(kp + 4 * E * c));
+    for (int c = 0; c < NKC; ++c) {
+      const T* kp = kl + (size_t)min(t0 + RC * c + lane / CR, t_end - 1) * kv_dim + col + E * (lane % CR);
+      kb[c] = __builtin_nontemporal_load(reinterpret_cast<const CT*>(kp));
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const T* vp = vl + (size_t)min(t0 + 4 * lk + r, t_end - 1) * kv_dim + col + 8 * li;
+      const T* vp = vl + (size_t)min(t0 + 4 * lk + r, t_end - 1) * kv_dim + col + E * li;
 #pragma unroll
       for (int h = 0; h < 8 / E; ++h)
-        vb[r * (8 / E) + h] = __builtin_nontemporal_load(reinterpret_cast<const CT*>(vp + E * h));
+        vb[r * (8 / E) + h] = __builtin_nontemporal_load(reinterpret_cast<const CT*>(vp + 64 * h));
     }
+  };
+  auto turn_k = [&](CT (&kb)[NKC]) {
+#pragma unroll
+    for (int c = 0; c < NKC; ++c) {
+      const int r = RC * c + lane / CR;
+      *reinterpret_cast<CT*>(turn + kRowB * r + 16 * ((lane % CR) ^ r)) = kb[c];
+    }
+#pragma unroll
+    for (int c = 0; c < NKC; ++c) kb[c] = *reinterpret_cast<const CT*>(turn + kRowB * li + 16 * ((lk + 4 * c) ^ li));
   };
   // q is scaled once the first tiles' loads are in flight (its own loads
   // then complete under theirs).
@@ -737,10 +782,12 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
         for (int h = 0; h < 8 / E; ++h)
           vb[r * (8 / E) + h] = *reinterpret_cast<const CT*>(base + kPlaneB + rv * kRowB +
-                                                             vq((8 * li + E * h) * (int)sizeof(T) / 16) * 16);
+                                                             vq((E * li + 64 * h) * (int)sizeof(T) / 16) * 16);
       }
     };
     if (n_steps > 0) {
+      turn_q();
+      __syncthreads();  // the ring's first stage overwrites the waves' q
       stage(0, 0);
       scale_q();
       for (int jt = 0; jt < n_steps; ++jt) {
@@ -759,11 +806,13 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
     for (int i = 0; i < D; ++i) load_tile(i, kr[i], vr[i]);
     __builtin_amdgcn_sched_barrier(0);
+    turn_q();
     scale_q();
     const int n_rounds = (my_tiles + D - 1) / D;
     for (int rr = 0; rr + 1 < n_rounds; ++rr) {
 #pragma unroll
       for (int i = 0; i < D; ++i) {
+        turn_k(kr[i]);
         compute(rr * D + i, kr[i], vr[i]);
         load_tile((rr + 1) * D + i, kr[i], vr[i]);
         __builtin_amdgcn_sched_barrier(0);
@@ -773,7 +822,10 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
       const int j0 = (n_rounds - 1) * D;
 #pragma unroll
       for (int i = 0; i < D; ++i)
-        if (j0 + i < my_tiles) compute(j0 + i, kr[i], vr[i]);
+        if (j0 + i < my_tiles) {
+          turn_k(kr[i]);
+          compute(j0 + i, kr[i], vr[i]);
+        }
     }
   }
   l_run = swap_sum<16>(l_run);
@@ -783,14 +835,15 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
     for (int b = 0; b < 8; ++b) o[b] *= 1.f / kPScale;  // the probabilities' scale, exactly
   }
-  // o[b][r] = O^T[d = 8*(4*lk + r) + b][m = li]. Merge the W waves in LDS.
+  // o[b][r] = O^T[d][m = li], d = E i + b % E + 64 (b / E) with i = 4 lk + r.
+  // Merge the W waves in LDS.
   auto sm_o = reinterpret_cast<float (*)[16][kD + 4]>(lds_raw);
   __shared__ float sm_ml[W][16][2];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    float* dst = &sm_o[wave][li][8 * (4 * lk + r)];
+    float* dst = &sm_o[wave][li][E * (4 * lk + r)];
     *reinterpret_cast<f32x4*>(dst) = f32x4{o[0][r], o[1][r], o[2][r], o[3][r]};
-    *reinterpret_cast<f32x4*>(dst + 4) = f32x4{o[4][r], o[5][r], o[6][r], o[7][r]};
+    *reinterpret_cast<f32x4*>(dst + (E == 4 ? 64 : 4)) = f32x4{o[4][r], o[5][r], o[6][r], o[7][r]};
   }
   if (lk == 0) {
     sm_ml[wave][li][0] = m_run;
