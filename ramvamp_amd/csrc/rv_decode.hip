@@ -451,7 +451,7 @@ __device__ __forceinline__ bool last_of(unsigned* t, unsigned n, int tid) {
 // element b of a lane's four V rows: the S^T accumulator is already the B
 // layout), and the output scaled back at the end; so the loads and the
 // output layout are the fp32 path's.
-template <typename T, int W, int D, bool PRO = false, bool H16 = false, bool LDS = false>
+template <typename T, int W, int D, bool PRO = false, bool H16 = false, bool LDS = false, bool TURN = true>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) void decode_tile_kernel(
     const float* __restrict__ q, PlanePtr<PRO, T> kl, PlanePtr<PRO, T> vl, int kv_dim, int positions, int split_len,
     int n_splits, int group, int kv_lo, float qscale, MergeArgs mg, float* __restrict__ out,
@@ -538,21 +538,29 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
   // one chunk fall on all banks. Against loads in operand order (per call,
   // one layer's graph, L2-resident up to 4096): f16 32768 positions 19.5 ->
   // 17.8 us, 2000 7.06 -> 6.89; fp32 16384 19.7 -> 17.8, 2000 8.35 -> 7.95, 400
-  // 7.06 -> 6.60; fp32 4096 the same; up to 100 positions +0.1-0.3 us where the
-  // rows are in the L2 (the turn-around's latency) and -0.1 where they are not.
+  // 7.06 -> 6.60; fp32 4096 the same. Where one workgroup per kv head takes all
+  // positions, a tile or two per wave, the turn-around's latency is what shows
+  // and the loads in operand order (!TURN) are the faster ones (plan_tile).
   char* const turn = lds_raw + (size_t)wave * (16 * (kD + 4) * (int)sizeof(float));
   float qv[32];
   // Row li of q: head li of the group (the first past it, unused). Loads of
   // 16 bytes at q's 4-byte alignment; two heads per load.
   typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
   f32x4a qr[8];
-  {
+  if constexpr (!TURN) {  // in operand order, 4-byte aligned
+    const float* qp = q + (size_t)(kvh * group + (col_ok ? li : 0)) * kD;
+#pragma unroll
+    for (int c = 0; c < NKC; ++c)
+#pragma unroll
+      for (int e = 0; e < E; ++e) qv[c * E + e] = qp[E * (lk + 4 * c) + e];
+  } else {
     const float* qp = q + (size_t)(kvh * group) * kD + 4 * (lane & 31);
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       if (2 * i < group) qr[i] = *reinterpret_cast<const f32x4a*>(qp + (size_t)min(2 * i + (lane >> 5), group - 1) * kD);
   }
   auto turn_q = [&]() {
+    if constexpr (!TURN) return;
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       if (2 * i < group) {
@@ -581,7 +589,8 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
     const int t0 = t_begin + (wave + j * W) * 16;
 #pragma unroll
     for (int c = 0; c < NKC; ++c) {
-      const T* kp = kl + (size_t)min(t0 + RC * c + lane / CR, t_end - 1) * kv_dim + col + E * (lane % CR);
+      const int row = TURN ? t0 + RC * c + lane / CR : t0 + li, chunk = TURN ? lane % CR : lk + 4 * c;
+      const T* kp = kl + (size_t)min(row, t_end - 1) * kv_dim + col + E * chunk;
       kb[c] = __builtin_nontemporal_load(reinterpret_cast<const CT*>(kp));
     }
 #pragma unroll
@@ -593,6 +602,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
   };
   auto turn_k = [&](CT (&kb)[NKC]) {
+    if constexpr (!TURN) return;
 #pragma unroll
     for (int c = 0; c < NKC; ++c) {
       const int r = RC * c + lane / CR;
@@ -1205,6 +1215,7 @@ constexpr int kTileWaves = 2048;
 struct TilePlan {
   int waves, depth, split_len, n_splits;
   int merge;  // MergeMode
+  bool turn;  // q and K loaded in row order and turned around in LDS
   bool lds;  // RV_TUNE_DECODE_IMPL 3: tiles staged through LDS (4 waves, depth 1)
 };
 
@@ -1284,6 +1295,13 @@ static TilePlan plan_tile(const rv_kv* kv, long positions) {
   p.depth = tile_depth(kv, p.waves, p.split_len, p.n_splits);
   p.lds = kv->tune_decode_impl == 3 && p.waves == 4;
   if (p.lds) p.depth = 1;
+  // One split per kv head: few loads per CU, each waited for, so q and K come
+  // in operand order without the turn through the LDS. 24-layer graphs, per
+  // call, turned vs operand order: f16 10 positions 3.75 vs 3.39 us, 64 3.89 vs
+  // 3.70, 100 4.79 vs 4.71, but 128 4.84 vs 4.94 and 190 5.94 vs 6.21; fp32 10
+  // 4.34 vs 3.98, 48 4.60 vs 4.58, 64 4.62 vs 4.73, 100 6.62 vs 6.20, 128 6.92
+  // vs 6.78 (its longest single split).
+  p.turn = p.n_splits > 1 || (kv->elem != RV_ELEM_F32 && positions > 112);
   p.merge = merge_mode(kv, p.n_splits);
   return p;
 }
@@ -1309,11 +1327,11 @@ static size_t tile_ws_bound(const rv_kv* kv, int n_heads, int group) {
   return (size_t)n_heads * (2 * (size_t)splits + 8) * part_stride_of(group);
 }
 
-template <typename T, int W, int D, bool PRO, bool H16, typename Pro>
+template <typename T, int W, int D, bool PRO, bool H16, bool TURN = true, typename Pro>
 static void launch_tile_wd(const TimedPair& tp, dim3 grid, hipStream_t s, const float* q, const void* kl,
                            const void* vl, int kv_dim, int positions, int split_len, int n_splits, int group,
                            int kv_lo, float qscale, const MergeArgs& mg, float* out, const Pro& pro) {
-  launch_timed(tp, decode_tile_kernel<T, W, D, PRO, H16>, grid, dim3(W * 64), s, q, (PlanePtr<PRO, T>)kl,
+  launch_timed(tp, decode_tile_kernel<T, W, D, PRO, H16, false, TURN>, grid, dim3(W * 64), s, q, (PlanePtr<PRO, T>)kl,
                (PlanePtr<PRO, T>)vl, kv_dim, positions, split_len, n_splits, group, kv_lo, qscale, mg, out, pro);
 }
 
@@ -1348,7 +1366,10 @@ static void launch_tile(const TilePlan& p, const TimedPair& tp, hipStream_t s, i
     else if (p.depth == 2) RV_TILE(1, 2);
     else RV_TILE(1, D4);
   } else {
-    if (p.depth == 1) RV_TILE(4, 1);
+    if (p.depth == 1 && !p.turn)
+      launch_tile_wd<T, 4, 1, PRO, H16, false>(tp, grid, s, q, kl, vl, kv_dim, positions, p.split_len, p.n_splits,
+                                               group, kv_lo, qscale, mg, out, pro);
+    else if (p.depth == 1) RV_TILE(4, 1);
     else if (p.depth == 2) RV_TILE(4, 2);
     else RV_TILE(4, D4);
   }

@@ -252,6 +252,27 @@ def test_decode_short_contexts_in_one_split(elem, lengths):
         gate(out, ref.attention(q, 0, scale, positions=p), what=f"{elem} positions {p}")
 
 
+@pytest.mark.parametrize("elem", ["f32", "f16"])
+@pytest.mark.parametrize("n_kv,group", [(4, 8), (1, 3), (2, 16), (3, 1)])
+def test_decode_on_both_sides_of_the_operand_order_loads(elem, n_kv, group):
+    # One split loads q and K in operand order (f16 up to 112 positions), the
+    # others in row order: tile edges on both sides, odd and full groups, with
+    # q at a 4-byte alignment; the gate is the file's.
+    torch = torch_cuda()
+    rng = Rng(0x0DE4 + 16 * n_kv + group)
+    kv, ref = twin_caches(rng, 1, n_kv, 128, 193, elem)
+    q = rng.vec_in(n_kv * group * 128, -1.0, 1.0)
+    dq = torch.zeros(q.size + 1, device="cuda")[1:]
+    dq.copy_(torch.from_numpy(q))
+    scale = np.float32(1.0) / np.sqrt(np.float32(128))
+    for p in (1, 15, 16, 17, 63, 112, 113, 128, 129, 192, 193):
+        say(f"case operand order {elem} n_kv={n_kv} group={group} positions={p}")
+        out = torch.full((q.size,), float("nan"), device="cuda")
+        rv.attention_at(dq, kv, 0, p, scale, None, out)
+        torch.cuda.synchronize()
+        gate(host(out), ref.attention(q, 0, scale, positions=p), what=f"{elem} positions {p}")
+
+
 @pytest.mark.parametrize("elem,n_pos,waves,split_len", [
     ("f32", 4096, 4, 0), ("f32", 4096, 2, 32), ("f32", 4096, 1, 16), ("f16", 32768, 4, 0), ("f16", 300, 4, 0),
     ("f32", 1000, 4, 64), ("f16", 20000, 1, 0), ("f32", 129, 1, 16), ("f16", 8193, 2, 0)])
