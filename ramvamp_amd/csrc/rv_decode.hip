@@ -533,7 +533,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
   // CU's address unit 64 cycles, one over consecutive lanes 16; the MFMA
   // operands of q and K have a row per lane. So the wave loads both in row
   // order and turns them around through its own part of the LDS (the bytes of
-  // its merge rows; a wave's LDS operations run in order, so no barrier), with
+  // its merge rows; a wave's LDS operations run in order: no barrier), with
   // a row's 16-byte chunks permuted by the row: 16 rows' writes and reads of
   // one chunk fall on all banks. Against loads in operand order (per call,
   // one layer's graph, L2-resident up to 4096): f16 32768 positions 19.5 ->
@@ -567,6 +567,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
         const int h = 2 * i + (lane >> 5);
         *reinterpret_cast<f32x4*>(turn + 512 * h + 16 * ((lane & 31) ^ h)) = qr[i];
       }
+    wave_lds_order();
     const int h = col_ok ? li : 0;
 #pragma unroll
     for (int c = 0; c < 8; ++c) {  // chunk of four: E = 4 takes lk + 4 c, E = 8 two of 2 (lk + 4 (c / 2))
@@ -575,6 +576,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
       for (int e = 0; e < 4; ++e) qv[4 * c + e] = v[e];
     }
+    wave_lds_order();  // read before a tile's K goes over it
   };
   // Rows past the split re-read its last row (in bounds, branch-free); their
   // scores are masked below, and tiles past the wave's share are loaded that
@@ -608,8 +610,10 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
       const int r = RC * c + lane / CR;
       *reinterpret_cast<CT*>(turn + kRowB * r + 16 * ((lane % CR) ^ r)) = kb[c];
     }
+    wave_lds_order();
 #pragma unroll
     for (int c = 0; c < NKC; ++c) kb[c] = *reinterpret_cast<const CT*>(turn + kRowB * li + 16 * ((lk + 4 * c) ^ li));
+    wave_lds_order();  // read before the next tile's K (or the merge rows) goes over it
   };
   // q is scaled once the first tiles' loads are in flight (its own loads
   // then complete under theirs).

@@ -155,6 +155,17 @@ __device__ __forceinline__ void load8(const _Float16* __restrict__ p, float (&x)
   for (int i = 0; i < 8; ++i) x[i] = (float)h[i];
 }
 
+// Orders the wave's LDS accesses before this point against those after it, for
+// lanes that read what other lanes of their wave wrote (or write over what
+// those read). The hardware runs a wave's LDS operations in order, so this
+// issues nothing: it keeps the compiler, which looks at one lane's addresses,
+// from moving one side over the other.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // 16 bytes per lane from global memory straight into LDS at the wave-uniform
 // base `l` + 16 * lane (global_load_lds_dwordx4). The device-only guard keeps
 // the host pass, which has no such builtin, from dropping the kernels' stubs.

@@ -273,6 +273,40 @@ def test_decode_on_both_sides_of_the_operand_order_loads(elem, n_kv, group):
         gate(host(out), ref.attention(q, 0, scale, positions=p), what=f"{elem} positions {p}")
 
 
+@pytest.mark.parametrize("elem", ["f32", "f16"])
+@pytest.mark.parametrize("n_kv,group,split_len", [(4, 8, 0), (4, 8, 320), (1, 3, 1024), (2, 16, 128)])
+def test_every_position_is_read_from_its_own_tile(elem, n_kv, group, split_len):
+    # q and K pass through the wave's LDS, one tile after another over the same
+    # bytes. Rows of K are random signs, so a query that is row t of K scores
+    # 128 there and at most 70 anywhere else (checked): its output is V's row t
+    # (the others' weights are below 2^-80), and a query or a tile read in place
+    # of another gives another row. Held to 2^-22 of the value, two ulps: the
+    # others still reach the MFMA's addition, which may take the last bit off.
+    # Splits of one to 16 tiles per wave, with a partial last tile.
+    torch = torch_cuda()
+    n = 4 * 320 + 327
+    say(f"case own tile {elem} n_kv={n_kv} group={group} split_len={split_len}")
+    rng = np.random.default_rng(0x711E + 64 * n_kv + group + split_len)
+    K = rng.choice(np.array([-1.0, 1.0], np.float32), (n, n_kv, 128))
+    V = ((2 * rng.integers(-512, 512, (n, n_kv, 128)) + 1) / 64).astype(np.float32)  # exact in f16, none 0
+    for h in range(n_kv):
+        near = K[:, h] @ K[:, h].T
+        np.fill_diagonal(near, 0.0)
+        assert near.max() <= 70.0
+    kv = rv.KvCache(1, n_kv, 128, n, elem)
+    kv.append_rows(0, K.reshape(n, -1), V.reshape(n, -1))
+    kv.set_tuning(rv.RV_TUNE_DECODE_SPLIT_LEN, split_len)
+    pick = rng.permutation(n)
+    pick = np.concatenate([pick, pick[:-n % group]]).reshape(-1, group)  # every position once
+    for at in pick:
+        q = np.stack([K[at, h] for h in range(n_kv)])  # head (h, g) asks for position at[g]
+        out = torch.empty(q.size, device="cuda")
+        rv.decode_attention(dev(q.ravel()), kv, 0, 1.0, None, out)
+        want = np.stack([V[at, h] for h in range(n_kv)])
+        off = np.abs(host(out).reshape(want.shape).astype(np.float64) - want) / np.abs(want)
+        assert off.max() <= 2.0 ** -22, f"positions {at}: {off.max():.2e}"
+
+
 @pytest.mark.parametrize("elem,n_pos,waves,split_len", [
     ("f32", 4096, 4, 0), ("f32", 4096, 2, 32), ("f32", 4096, 1, 16), ("f16", 32768, 4, 0), ("f16", 300, 4, 0),
     ("f32", 1000, 4, 64), ("f16", 20000, 1, 0), ("f32", 129, 1, 16), ("f16", 8193, 2, 0)])
