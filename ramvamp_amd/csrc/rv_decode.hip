@@ -538,9 +538,9 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
   // one chunk fall on all banks. Against loads in operand order (per call,
   // one layer's graph, L2-resident up to 4096): f16 32768 positions 19.5 ->
   // 17.8 us, 2000 7.06 -> 6.89; fp32 16384 19.7 -> 17.8, 2000 8.35 -> 7.95, 400
-  // 7.06 -> 6.60; fp32 4096 the same. Where one workgroup per kv head takes all
-  // positions, a tile or two per wave, the turn-around's latency is what shows
-  // and the loads in operand order (!TURN) are the faster ones (plan_tile).
+  // 7.06 -> 6.60; fp32 4096 the same. With few positions a call the turn-around's
+  // latency is what shows, and the loads in operand order (!TURN) are the faster
+  // ones (turned).
   char* const turn = lds_raw + (size_t)wave * (16 * (kD + 4) * (int)sizeof(float));
   float qv[32];
   // Row li of q: head li of the group (the first past it, unused). Loads of
@@ -1219,7 +1219,6 @@ constexpr int kTileWaves = 2048;
 struct TilePlan {
   int waves, depth, split_len, n_splits;
   int merge;  // MergeMode
-  bool turn;  // q and K loaded in row order and turned around in LDS
   bool lds;  // RV_TUNE_DECODE_IMPL 3: tiles staged through LDS (4 waves, depth 1)
 };
 
@@ -1299,15 +1298,28 @@ static TilePlan plan_tile(const rv_kv* kv, long positions) {
   p.depth = tile_depth(kv, p.waves, p.split_len, p.n_splits);
   p.lds = kv->tune_decode_impl == 3 && p.waves == 4;
   if (p.lds) p.depth = 1;
-  // One split per kv head: few loads per CU, each waited for, so q and K come
-  // in operand order without the turn through the LDS. 24-layer graphs, per
-  // call, turned vs operand order: f16 10 positions 3.75 vs 3.39 us, 64 3.89 vs
-  // 3.70, 100 4.79 vs 4.71, but 128 4.84 vs 4.94 and 190 5.94 vs 6.21; fp32 10
-  // 4.34 vs 3.98, 48 4.60 vs 4.58, 64 4.62 vs 4.73, 100 6.62 vs 6.20, 128 6.92
-  // vs 6.78 (its longest single split).
-  p.turn = p.n_splits > 1 || (kv->elem != RV_ELEM_F32 && positions > 112);
   p.merge = merge_mode(kv, p.n_splits);
   return p;
+}
+
+// Whether the default form (4 waves, one tile at a time) loads q and K in row
+// order and turns them around in LDS. With few positions each load is waited
+// for and the turn's latency shows; with more, the address unit's cycles do.
+// 24-layer graphs, us per call, turned vs operand order (medians of three):
+//  - f16 MFMA operands: 10 positions 3.71 vs 3.41, 64 3.87 vs 3.72, 128 4.57 vs
+//    4.39, 190 5.13 vs 4.94, 256 5.87 vs 5.69, 384 5.90 vs 5.78, 512 5.92 vs
+//    5.93, 600 6.73 vs 6.82, 1000 6.84 vs 6.99;
+//  - fp32 operands, fp32 planes: one split (up to 128 positions) 10 4.39 vs
+//    4.03, 48 4.62 vs 4.59, 100 6.54 vs 6.19, 128 6.42 vs 6.24 (64 alone, every
+//    wave with one whole tile, is the other way: 4.64 vs 4.83); several splits
+//    144 6.53 vs 6.77, 256 6.52 vs 6.75;
+//  - with the step's prologue: f16 planes 128 8.84 vs 9.16, 300 8.79 vs 8.88
+//    (11 6.87 vs 6.83; 101 8.78 vs 8.90, left with the shorter ones), fp32 191
+//    8.47 vs 8.62 (11 6.51 vs 6.03, 101 8.63 vs 8.55; 128 8.66 vs 8.82).
+template <typename T, bool H16>
+static bool turned(const TilePlan& p, int positions) {
+  if (H16) return positions > 512;
+  return p.n_splits > 1 || (!std::is_same<T, float>::value && positions > 112);
 }
 
 // Workspace floats of a plan: level-1 rows, then level-2 rows.
@@ -1370,7 +1382,7 @@ static void launch_tile(const TilePlan& p, const TimedPair& tp, hipStream_t s, i
     else if (p.depth == 2) RV_TILE(1, 2);
     else RV_TILE(1, D4);
   } else {
-    if (p.depth == 1 && !p.turn)
+    if (p.depth == 1 && !turned<T, H16>(p, positions))
       launch_tile_wd<T, 4, 1, PRO, H16, false>(tp, grid, s, q, kl, vl, kv_dim, positions, p.split_len, p.n_splits,
                                                group, kv_lo, qscale, mg, out, pro);
     else if (p.depth == 1) RV_TILE(4, 1);

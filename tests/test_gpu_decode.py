@@ -273,6 +273,22 @@ def test_decode_on_both_sides_of_the_operand_order_loads(elem, n_kv, group):
         gate(host(out), ref.attention(q, 0, scale, positions=p), what=f"{elem} positions {p}")
 
 
+@pytest.mark.parametrize("n_kv,group", [(4, 8), (1, 3)])
+def test_decode_on_both_sides_of_512_positions(n_kv, group):
+    # f16 MFMA operands are loaded in operand order up to 512 positions and in
+    # row order from there; the gate is the file's.
+    torch_cuda()
+    rng = Rng(0x0512 + group)
+    kv, ref = twin_caches(rng, 1, n_kv, 128, 529, "f16")
+    q = rng.vec_in(n_kv * group * 128, -1.0, 1.0)
+    scale = np.float32(1.0) / np.sqrt(np.float32(128))
+    for p in (193, 496, 512, 513, 529):
+        say(f"case 512 n_kv={n_kv} group={group} positions={p}")
+        out = dev(np.full(q.size, np.nan))
+        rv.attention_at(dev(q), kv, 0, p, scale, None, out)
+        gate(host(out), ref.attention(q, 0, scale, positions=p), what=f"positions {p}")
+
+
 @pytest.mark.parametrize("elem", ["f32", "f16"])
 @pytest.mark.parametrize("n_kv,group,split_len", [(4, 8, 0), (4, 8, 320), (1, 3, 1024), (2, 16, 128)])
 def test_every_position_is_read_from_its_own_tile(elem, n_kv, group, split_len):
