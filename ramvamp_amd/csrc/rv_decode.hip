@@ -451,7 +451,7 @@ __device__ __forceinline__ bool last_of(unsigned* t, unsigned n, int tid) {
 // element b of a lane's four V rows: the S^T accumulator is already the B
 // layout), and the output scaled back at the end; so the loads and the
 // output layout are the fp32 path's.
-template <typename T, int W, int D, bool PRO = false, bool H16 = false, bool LDS = false, bool TURN = true>
+template <typename T, int W, int D, bool PRO, bool H16, bool LDS, bool TURN>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) void decode_tile_kernel(
     const float* __restrict__ q, PlanePtr<PRO, T> kl, PlanePtr<PRO, T> vl, int kv_dim, int positions, int split_len,
     int n_splits, int group, int kv_lo, float qscale, MergeArgs mg, float* __restrict__ out,
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
   // The LDS form stages 64-position tiles (16 positions per wave) of K and V
   // for the whole workgroup, two stages of kStage bytes; the waves' merge
   // below reuses the same bytes once the ring is drained.
-  static_assert(!LDS || (W == 4 && D == 1 && !PRO), "LDS staging: 4 waves, one tile per step, no prologue");
+  static_assert(!LDS || (W == 4 && D == 1 && !PRO && !TURN), "LDS staging: 4 waves, one tile per step, no prologue");
   constexpr int kRowB = kD * (int)sizeof(T);  // bytes of one position's head slice
   constexpr int kPlaneB = 64 * kRowB;         // one plane of a staged tile
   constexpr int kStage = 2 * kPlaneB;
@@ -765,13 +765,12 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
     // Staged form: step jt's 64 positions (wave w computes the 16 at 16 w)
     // land in LDS by direct-to-LDS loads, each 1 KiB piece from one wave,
     // while the previous step is computed. Row r's 16-byte K chunks are
-    // stored XOR-permuted by r % 16 and V's (fp32) with bit 4 of the chunk
-    // folded into bit 0, so the operand reads below are free of bank
-    // conflicts; the operands and their clamping are the register form's.
+    // stored XOR-permuted by r % 16, so that the operand reads below are free
+    // of bank conflicts (V's read consecutive chunks as they are); the operands
+    // and their clamping are the register form's.
     constexpr int kLPW = kStage / 1024 / W;  // pieces per wave per stage
     const int n_steps = (n_tiles + W - 1) / W;
     auto kq = [](int r, int q) { return q ^ (r & 15); };
-    auto vq = [](int q) { return sizeof(T) == 4 ? q ^ ((q >> 4) & 1) : q; };
     auto stage = [&](int jt, int st) {
       jt = min(jt, n_steps - 1);  // past the last step: the last again (never read)
 #pragma unroll
@@ -781,7 +780,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
         const int r = ob / kRowB, q = (ob % kRowB) / 16;
         const int t = min(t_begin + 64 * jt + r, t_end - 1);
         const T* src = (plane == 0 ? kl + (size_t)t * kv_dim + col + kq(r, q) * (16 / (int)sizeof(T))
-                                   : vl + (size_t)t * kv_dim + col + vq(q) * (16 / (int)sizeof(T)));
+                                   : vl + (size_t)t * kv_dim + col + q * (16 / (int)sizeof(T)));
         lds_load16(src, (lds_void*)(lds_raw + st * kStage + piece * 1024));
       }
     };
@@ -795,13 +794,11 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2))) voi
         const int rv = 16 * wave + 4 * lk + r;
 #pragma unroll
         for (int h = 0; h < 8 / E; ++h)
-          vb[r * (8 / E) + h] = *reinterpret_cast<const CT*>(base + kPlaneB + rv * kRowB +
-                                                             vq((E * li + 64 * h) * (int)sizeof(T) / 16) * 16);
+          vb[r * (8 / E) + h] =
+              *reinterpret_cast<const CT*>(base + kPlaneB + rv * kRowB + (E * li + 64 * h) * (int)sizeof(T));
       }
     };
     if (n_steps > 0) {
-      turn_q();
-      __syncthreads();  // the ring's first stage overwrites the waves' q
       stage(0, 0);
       scale_q();
       for (int jt = 0; jt < n_steps; ++jt) {
@@ -1343,7 +1340,7 @@ static size_t tile_ws_bound(const rv_kv* kv, int n_heads, int group) {
   return (size_t)n_heads * (2 * (size_t)splits + 8) * part_stride_of(group);
 }
 
-template <typename T, int W, int D, bool PRO, bool H16, bool TURN = true, typename Pro>
+template <typename T, int W, int D, bool PRO, bool H16, bool TURN, typename Pro>
 static void launch_tile_wd(const TimedPair& tp, dim3 grid, hipStream_t s, const float* q, const void* kl,
                            const void* vl, int kv_dim, int positions, int split_len, int n_splits, int group,
                            int kv_lo, float qscale, const MergeArgs& mg, float* out, const Pro& pro) {
@@ -1358,36 +1355,42 @@ static void launch_tile(const TilePlan& p, const TimedPair& tp, hipStream_t s, i
   const dim3 grid((unsigned)(n_heads * p.n_splits));
   if constexpr (!PRO) {
     if (p.lds) {
-      launch_timed(tp, decode_tile_kernel<T, 4, 1, false, H16, true>, grid, dim3(256), s, q, (PlanePtr<false, T>)kl,
+      launch_timed(tp, decode_tile_kernel<T, 4, 1, false, H16, true, false>, grid, dim3(256), s, q, (PlanePtr<false, T>)kl,
                    (PlanePtr<false, T>)vl, kv_dim, positions, p.split_len, p.n_splits, group, kv_lo, qscale, mg, out,
                    pro);
       return;
     }
   }
-#define RV_TILE(W, D)                                                                                              \
-  launch_tile_wd<T, W, D, PRO, H16>(tp, grid, s, q, kl, vl, kv_dim, positions, p.split_len, p.n_splits, group, kv_lo, \
-                                    qscale, mg, out, pro)
+#define RV_TILE(W, D, TURN)                                                                                  \
+  launch_tile_wd<T, W, D, PRO, H16, TURN>(tp, grid, s, q, kl, vl, kv_dim, positions, p.split_len, p.n_splits, \
+                                          group, kv_lo, qscale, mg, out, pro)
+  // Which tuned forms turn q and K around in LDS, by time over the same form
+  // before it did (100 / 2000 / 16384 positions, default splits; then splits of
+  // 1024 at 16384). 8 waves: f16 1.00 / 0.93 / 0.90; 0.82, fp32 0.93 / 0.88 /
+  // 0.98; 0.70. 4 waves, depth 2 and 4: f16 1.01 / 1.01 / 0.95; 0.81, fp32 0.91 /
+  // 0.95 / 0.95; 0.71. Not 1 or 2: turned, f16 1 wave 1.07 / 1.06 / 1.04; 1.19,
+  // 2 waves 1.07 / 1.04 / 1.01; 0.94, fp32 1 wave 1.06 / 1.12 / 1.19; 1.20 and
+  // spilled registers at depth 2, 2 waves 1.03 / 1.05 / 0.97; 1.07, where in
+  // operand order they are at 0.93-1.01 throughout.
   // Depth 4 only for f16 planes (fp32 tiles would spill).
   constexpr int D4 = std::is_same<T, float>::value ? 2 : 4;
   if (p.waves == 8) {
-    if (p.depth == 1) RV_TILE(8, 1);
-    else if (p.depth == 2) RV_TILE(8, 2);
-    else RV_TILE(8, D4);
+    if (p.depth == 1) RV_TILE(8, 1, true);
+    else if (p.depth == 2) RV_TILE(8, 2, true);
+    else RV_TILE(8, D4, true);
   } else if (p.waves == 2) {
-    if (p.depth == 1) RV_TILE(2, 1);
-    else if (p.depth == 2) RV_TILE(2, 2);
-    else RV_TILE(2, D4);
+    if (p.depth == 1) RV_TILE(2, 1, false);
+    else if (p.depth == 2) RV_TILE(2, 2, false);
+    else RV_TILE(2, D4, false);
   } else if (p.waves == 1) {
-    if (p.depth == 1) RV_TILE(1, 1);
-    else if (p.depth == 2) RV_TILE(1, 2);
-    else RV_TILE(1, D4);
+    if (p.depth == 1) RV_TILE(1, 1, false);
+    else if (p.depth == 2) RV_TILE(1, 2, false);
+    else RV_TILE(1, D4, false);
   } else {
-    if (p.depth == 1 && !turned<T, H16>(p, positions))
-      launch_tile_wd<T, 4, 1, PRO, H16, false>(tp, grid, s, q, kl, vl, kv_dim, positions, p.split_len, p.n_splits,
-                                               group, kv_lo, qscale, mg, out, pro);
-    else if (p.depth == 1) RV_TILE(4, 1);
-    else if (p.depth == 2) RV_TILE(4, 2);
-    else RV_TILE(4, D4);
+    if (p.depth == 1 && !turned<T, H16>(p, positions)) RV_TILE(4, 1, false);
+    else if (p.depth == 1) RV_TILE(4, 1, true);
+    else if (p.depth == 2) RV_TILE(4, 2, true);
+    else RV_TILE(4, D4, true);
   }
 #undef RV_TILE
 }
