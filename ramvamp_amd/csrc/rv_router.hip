@@ -231,8 +231,7 @@ __global__ __launch_bounds__(kRouterThreads) void router_kernel(const float* __r
       prob[be] = -INFINITY;
     }
     s += bp;  // the selection-order f32 sum, identical on every lane
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    wave_lds_order();  // lane 0's -inf before the next round's reads
   }
   if (norm && lane == 0) {
     for (int k = 0; k < top_k; ++k) wo[k] = wo[k] / s;
@@ -329,7 +328,7 @@ __device__ __forceinline__ void choose(StagedLds<R>& s, int r, int lane, int n_e
     e[h] = exp((double)p[h] - m);
     s.ex[r][lane + 64 * h] = lane + 64 * h < n_experts ? e[h] : 0.0;
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_order();  // the other lanes' exponentials below
   // The sum in expert order (every lane the same); slots past n_experts hold
   // +0, which leaves a sum of exponentials as it is.
   double sum = 0.0;
