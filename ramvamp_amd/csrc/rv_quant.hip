@@ -412,11 +412,6 @@ __global__ __launch_bounds__(64 * kRowsPerWG) void gemv_rows_kernel(const uint8_
   if (lane == 0) out[i] = v;
 }
 
-// The fused projections: one row per wave, 8 waves per workgroup, the f32
-// activation row quantized once per workgroup into LDS first (the same
-// per-block code as the quantizer kernels, so bit-identical), then every
-// wave's GEMV row reads its blocks from LDS. Segments (at most 3) are row
-// ranges of independent matrices, each against the Q8_K or the Q8_0 form.
 // 1 / sqrt(mean(x^2) + eps) of n values, as norm.rs:18-26 computes it: the
 // squares summed in f64 (here per thread, then over lanes and waves in a
 // fixed order, so every thread of the workgroup gets the same value), sqrt
@@ -451,18 +446,20 @@ __device__ __forceinline__ double wave_sum_tree_f64(double x) {
   return x;
 }
 
-// One wave's part of a fused projection: its weight row (FMT) is loaded while
-// the workgroup (normalizes and) quantizes x; NB Q8_K blocks of x per wave.
-// Every wave of the workgroup comes through here, each with its row's FMT, and
-// passes the same barriers; a wave past the last row has live false.
+// One workgroup of a fused projection, eight rows of a segment, one per wave:
+// the wave's weight row is loaded while the workgroup (normalizes and)
+// quantizes x into LDS, NB 256-value blocks of x per wave, in the form that FMT
+// takes (the same per-block code as the quantizer kernels, so bit-identical).
+// All rows of a workgroup are of one segment, so its waves run one FMT and pass
+// the same barriers; a wave past the segment's last row has live false.
 template <int FMT, bool NORM, int NB>
-__device__ __forceinline__ void fused_wave(const FusedProjArgs& a, const FusedSeg& s, int i, bool live, bool need_k,
-                                           bool need_0, int wave, int lane, rv_block_q8_k* lk, rv_block_q8_0* l0,
-                                           double* red) {
+__device__ __forceinline__ void fused_rows(const FusedProjArgs& a, const FusedSeg& s, int i, bool live, int wave,
+                                           int lane, void* lds, double* red) {
 #pragma clang fp contract(off)
   typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
   constexpr int P = FMT != RV_QF_Q8_0 && NB > 1 ? 2 : 1;  // passes whose weights are loaded ahead
-  const int nbw = FMT == RV_QF_Q8_0 ? a.nb0 : a.nbk;
+  constexpr bool kQ80 = FMT == RV_QF_Q8_0;
+  const int nbw = kQ80 ? a.nb0 : a.nbk;
   // The lane's four values of each of the wave's blocks (blocks past the row
   // re-read its last), straight into the quantizers' registers; with the norm
   // also its weight and, for the sum of squares, the values in the summing
@@ -513,56 +510,47 @@ __device__ __forceinline__ void fused_wave(const FusedProjArgs& a, const FusedSe
     float v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = NORM ? xv[u][e] * inv * wv[u][e] : xv[u][e];
-    if (need_k) store_q8_k(quantize_lane_q8_k(v), &lk[b], lane);
-    if (need_0) {
+    if constexpr (kQ80) {
       const Q80Lane z = quantize_lane_q8_0(v);
-      rv_block_q8_0* blk = &l0[8 * b + (lane >> 3)];
+      rv_block_q8_0* blk = reinterpret_cast<rv_block_q8_0*>(lds) + 8 * b + (lane >> 3);
       *reinterpret_cast<uint32_t*>(blk->qs + 4 * (lane & 7)) = z.q;
       if ((lane & 7) == 0) blk->d = z.d;
+    } else {
+      store_q8_k(quantize_lane_q8_k(v), reinterpret_cast<rv_block_q8_k*>(lds) + b, lane);
     }
   }
   __syncthreads();
   if (!live || gate > a.gate_max) return;  // (the whole grid's decode step was refused: nothing is written)
-  const float v = row_sum<FMT, P>(pre, row, nbw, FMT == RV_QF_Q8_0 ? (const void*)l0 : (const void*)lk, lane);
+  const float v = row_sum<FMT, P>(pre, row, nbw, lds, lane);
   if (lane == 0) s.out[i] = s.add ? addv + v : v;
 }
 
-// NB: Q8_K blocks per wave (x holds at most 256 * kFusedWaves * NB values).
+// Workgroups of a segment of n rows.
+__host__ __device__ constexpr int fused_groups(int n) { return (n + kFusedWaves - 1) / kFusedWaves; }
+
+// NB: 256-value blocks per wave (x holds at most 256 * kFusedWaves * NB values).
 template <bool NORM, int NB>
 __global__ __launch_bounds__(64 * kFusedWaves) void fused_proj_kernel(FusedProjArgs a) {
-  __shared__ rv_block_q8_k lk[kFusedWaves * NB];
-  __shared__ rv_block_q8_0 l0[kFusedWaves * NB * 8];
+  // x as Q8_K blocks or as eight times as many Q8_0 blocks.
+  static_assert(sizeof(rv_block_q8_k) >= 8 * sizeof(rv_block_q8_0), "the Q8_0 form fits the Q8_K form's bytes");
+  __shared__ rv_block_q8_k lds[kFusedWaves * NB];
   __shared__ double red[kFusedWaves];
   // The wave index as a scalar: the row, its segment and the segment's
   // fields are then wave-uniform, read with scalar loads from the kernel
   // arguments (indexed from a vector register, each was a vector load of
   // the argument segment that every later load waited behind).
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int first = (int)blockIdx.x * kFusedWaves;
-  // The segments this workgroup's rows touch decide which forms it needs.
-  bool need_k = false, need_0 = false;
-  {
-    int lo = 0;
-    for (int sg = 0; sg < a.n_seg; ++sg) {
-      const int hi = lo + a.n_rows[sg];
-      if (first < hi && first + kFusedWaves > lo) (a.seg[sg].fmt == RV_QF_Q8_0 ? need_0 : need_k) = true;
-      lo = hi;
-    }
-  }
-  int i = first + wave, sg = 0;
-  while (sg < a.n_seg && i >= a.n_rows[sg]) i -= a.n_rows[sg++];
-  const bool live = sg < a.n_seg;
-  if (!live) {  // past the last row: quantizes beside the others, on the last segment that has rows
-    sg = a.n_seg - 1;
-    while (a.n_rows[sg] == 0) --sg;
-    i = a.n_rows[sg] - 1;
-  }
+  int b = (int)blockIdx.x, sg = 0;
+  while (sg + 1 < a.n_seg && b >= fused_groups(a.n_rows[sg])) b -= fused_groups(a.n_rows[sg++]);
+  const bool live = b * kFusedWaves + wave < a.n_rows[sg];
+  // A wave past the last row quantizes beside the others, on that row's bytes.
+  const int i = min(b * kFusedWaves + wave, a.n_rows[sg] - 1);
   const FusedSeg& s = a.seg[sg];
-  switch (s.fmt) {
-    case RV_QF_Q4_K: return fused_wave<RV_QF_Q4_K, NORM, NB>(a, s, i, live, need_k, need_0, wave, lane, lk, l0, red);
-    case RV_QF_Q5_K: return fused_wave<RV_QF_Q5_K, NORM, NB>(a, s, i, live, need_k, need_0, wave, lane, lk, l0, red);
-    case RV_QF_Q6_K: return fused_wave<RV_QF_Q6_K, NORM, NB>(a, s, i, live, need_k, need_0, wave, lane, lk, l0, red);
-    default: return fused_wave<RV_QF_Q8_0, NORM, NB>(a, s, i, live, need_k, need_0, wave, lane, lk, l0, red);
+  switch (s.fmt) {  // workgroup-uniform
+    case RV_QF_Q4_K: return fused_rows<RV_QF_Q4_K, NORM, NB>(a, s, i, live, wave, lane, lds, red);
+    case RV_QF_Q5_K: return fused_rows<RV_QF_Q5_K, NORM, NB>(a, s, i, live, wave, lane, lds, red);
+    case RV_QF_Q6_K: return fused_rows<RV_QF_Q6_K, NORM, NB>(a, s, i, live, wave, lane, lds, red);
+    default: return fused_rows<RV_QF_Q8_0, NORM, NB>(a, s, i, live, wave, lane, lds, red);
   }
 }
 
@@ -714,10 +702,10 @@ HipStatus launch_fill_zero(float* out, size_t n, hipStream_t s) {
 
 HipStatus launch_fused_proj(const FusedProjArgs& a, hipStream_t s) {
   HipStatus st;
-  long rows = 0;
-  for (int i = 0; i < a.n_seg; ++i) rows += a.n_rows[i];
-  if (rows == 0) return st;
-  const dim3 grid((unsigned)((rows + kFusedWaves - 1) / kFusedWaves)), block(64 * kFusedWaves);
+  unsigned groups = 0;
+  for (int i = 0; i < a.n_seg; ++i) groups += (unsigned)fused_groups(a.n_rows[i]);
+  if (groups == 0) return st;
+  const dim3 grid(groups), block(64 * kFusedWaves);
 #define RV_FUSED(NB)                                                          \
   if (a.norm_w)                                                               \
     hipLaunchKernelGGL((fused_proj_kernel<true, NB>), grid, block, 0, s, a);  \

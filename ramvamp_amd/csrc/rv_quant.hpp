@@ -10,15 +10,15 @@ namespace rv {
 
 // The fused projections (one launch): up to three row ranges of
 // independent matrices, each against the Q8_K (k-quant formats) or the Q8_0
-// (RV_QF_Q8_0) form of one f32 activation row x, which each workgroup
-// quantizes into LDS before its rows run. x holds nbk * 256 = nb0 * 32
-// values, at most kFusedMaxKBlocks * 256.
+// (RV_QF_Q8_0) form of one f32 activation row x, which each workgroup (eight
+// rows of one range) quantizes into LDS before its rows run. x holds nbk * 256
+// = nb0 * 32 values, at most kFusedMaxKBlocks * 256.
 constexpr int kFusedWaves = 8;
 constexpr int kFusedMaxKBlocks = 32;
 constexpr int kFusedMax0Blocks = kFusedMaxKBlocks * 8;
 // With norm_w set, x is first RMS-normalized (norm.rs:18-58: f64 mean of
-// squares, x * inv * w in f32) in LDS, and the normalized row is what gets
-// quantized. With a segment's `add` set, its rows store add[i] + dot
+// squares, x * inv * w in f32) in registers, and the normalized row is what
+// gets quantized. With a segment's `add` set, its rows store add[i] + dot
 // (vec.rs:10-22; add may alias out).
 struct FusedSeg {
   uint32_t fmt;

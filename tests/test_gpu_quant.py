@@ -246,3 +246,27 @@ def test_projections_quantize_in_the_wave_like_the_quantizers():
     o = torch.empty(kv_dim, device="cuda")
     P.attn_out_proj(f32(torch, x), oracle.RV_QF_Q5_K, u8(torch, wo), o)
     assert o.cpu().numpy().tobytes() == oracle.gemv(oracle.RV_QF_Q5_K, wo, hidden, kv_dim, acts_k).tobytes()
+
+
+@pytest.mark.parametrize("hidden", [256, 2304, 8192])
+@pytest.mark.parametrize("q_dim,kv_dim", [(1, 1), (9, 3), (17, 8), (23, 42)])
+def test_fused_projections_at_ragged_row_counts(hidden, q_dim, kv_dim):
+    """Row counts around the eight rows of a workgroup: each range's last
+    workgroup is partial, and the next range, of another format, starts in a
+    workgroup of its own. Bit-identical to quantize-then-GEMV."""
+    torch = torch_cuda()
+    rng = np.random.default_rng(0x8A9 + hidden + 64 * q_dim + kv_dim)
+    x = rng.standard_normal(hidden).astype(F32)
+    acts_k, acts_0 = oracle.quantize_row_q8_k(x), oracle.quantize_row_q8_0(x)
+    for q_fmt, v_fmt in ((FORMATS[0], FORMATS[1]), (FORMATS[1], FORMATS[2]), (FORMATS[2], FORMATS[0])):
+        say(f"case ragged projections hidden={hidden} q={q_dim} kv={kv_dim} formats {q_fmt} {v_fmt}")
+        wq, wk, wv = (random_weight_rows(f, m, hidden, rng)
+                      for f, m in ((q_fmt, q_dim), (oracle.RV_QF_Q8_0, kv_dim), (v_fmt, kv_dim)))
+        q, k, v = (torch.full((m,), float("nan"), device="cuda") for m in (q_dim, kv_dim, kv_dim))
+        P.attn_in_proj(f32(torch, x), q_fmt, u8(torch, wq), q, u8(torch, wk), k, v_fmt, u8(torch, wv), v)
+        o = torch.full((kv_dim,), float("nan"), device="cuda")
+        P.attn_out_proj(f32(torch, x), v_fmt, u8(torch, wv), o)
+        assert q.cpu().numpy().tobytes() == oracle.gemv(q_fmt, wq, hidden, q_dim, acts_k).tobytes()
+        assert k.cpu().numpy().tobytes() == oracle.gemv(oracle.RV_QF_Q8_0, wk, hidden, kv_dim, acts_0).tobytes()
+        want = oracle.gemv(v_fmt, wv, hidden, kv_dim, acts_k).tobytes()
+        assert v.cpu().numpy().tobytes() == want and o.cpu().numpy().tobytes() == want
