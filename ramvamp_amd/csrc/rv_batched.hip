@@ -38,9 +38,12 @@
 // Loads go to consecutive lanes at dword-aligned addresses: a 64-lane load
 // whose neighbouring lanes fall into different rows takes 64 cycles of the
 // CU's address unit whatever its width, and one of 16 bytes a lane at odd
-// 2-byte offsets 140-280, against 16 for 1 KiB contiguous. The activations
-// come in operand order from the rows quantizer (PackedActs, rv_quant.hpp),
-// 1 KiB contiguous per load.
+// 2-byte offsets 140-280, against 16 for 1 KiB contiguous. A prefill chunk's
+// activations come in operand order from the rows quantizer (PackedActs,
+// rv_quant.hpp), 1 KiB contiguous per load; those of the public calls are blocks
+// row by row, turned around on the way (TurnedActs) unless they are few.
+#include <type_traits>
+
 #include "rv_device.hpp"
 #include "rv_internal.hpp"
 #include "rv_quant.hpp"
@@ -52,12 +55,8 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 // Global accesses at the alignment the packed rows have (2 or 4 bytes).
 typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint32_t u32x4h __attribute__((ext_vector_type(4), aligned(2)));
-typedef uint32_t u32x2h __attribute__((ext_vector_type(2), aligned(2)));
-typedef uint32_t u32x2a __attribute__((ext_vector_type(2), aligned(4)));
 typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
 typedef _Float16 f16x4a __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -247,83 +246,184 @@ struct Act {
   float d[FMT == RV_QF_Q8_0 ? 8 : 1];
 };
 
-// Where a lane finds its tile's operands: the tile's (packed) or the first
-// row's (public) bytes, wave-uniform, and the lane's offsets from there.
+// How a wave gets its activation tile, one block (Q8_0: a group of eight) after
+// another: packed operands as they are; public blocks in operand order straight
+// from memory (k-quants); or public blocks turned around in LDS (TurnedActs).
+enum ActSrc { kPacked, kDirect, kTurned };
+
+// Packed and direct: where a lane finds its tile's operands, the tile's (packed)
+// or its first row's bytes, wave-uniform, and the lane's offsets from there. The
+// next block's are loaded while one is used.
 struct ActAt {
   const char* base;
   int nt, step;  // step: bytes to the next block
   uint32_t q, bs, d;
 };
 
-template <int FMT, bool PACKED>
+template <int FMT, int SRC>
 __device__ __forceinline__ ActAt act_at(const BatchedArgs& a, int tile, int col, int kq) {
   constexpr bool kQ80 = FMT == RV_QF_Q8_0;
+  static_assert(SRC == kPacked || (SRC == kDirect && !kQ80), "packed, or public k-quants");
+  constexpr int kUnit = kQ80 ? kPacked0Bytes : kPackedKBytes;  // also a public block's size (k-quants)
   const char* acts = reinterpret_cast<const char*>(kQ80 ? a.acts_0 : a.acts_k);
   const int left = a.n_acts - 16 * tile;
   ActAt r;
   r.nt = min(16, left);
   const uint32_t i = (uint32_t)min(col, r.nt - 1);
-  if constexpr (PACKED) {
-    constexpr int kUnit = kQ80 ? kPacked0Bytes : kPackedKBytes;
-    r.base = acts + (size_t)tile * 16 * (a.in_dim / 256) * kUnit;
+  r.base = acts + (size_t)tile * 16 * (a.in_dim / 256) * kUnit;
+  if constexpr (SRC == kPacked) {
     r.step = r.nt * kUnit;
     r.q = ((uint32_t)kq * r.nt + i) * 16;
     r.bs = 256 * r.nt + ((uint32_t)kq * r.nt + i) * 8;
     r.d = kQ80 ? 256 * r.nt + 32 * i : 288 * r.nt + 4 * i;
   } else {
-    const size_t row = kQ80 ? (size_t)(a.in_dim / 32) * sizeof(rv_block_q8_0) : (size_t)(a.in_dim / 256) * sizeof(rv_block_q8_k);
-    r.base = acts + (size_t)(16 * tile + i) * row;  // the lane's own row
-    r.q = r.bs = r.d = 0;
-    r.step = kQ80 ? 0 : (int)sizeof(rv_block_q8_k);  // Q8_0: load_act's step
+    r.step = kUnit;
+    r.d = i * (uint32_t)(a.in_dim / 256) * kUnit;  // the lane's own row
+    r.q = r.d + 4 + 16 * kq;
+    r.bs = 0;
   }
   return r;
 }
 
-template <int FMT, bool PACKED>
-__device__ __forceinline__ void load_act(Act<FMT>& y, const ActAt& at, int nb, int step, int kq) {
-  constexpr bool kQ80 = FMT == RV_QF_Q8_0;
-  if constexpr (PACKED) {
-    const char* base = at.base;
+template <int FMT, int SRC>
+__device__ __forceinline__ void load_act(Act<FMT>& y, const ActAt& at) {
+  const char* base = at.base;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const u32x4a v = *reinterpret_cast<const u32x4a*>(base + 64 * c * at.nt + at.q);
-      y.q[c] = i32x4{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
-    }
-    if constexpr (kQ80) {
-      const f32x4a d0 = *reinterpret_cast<const f32x4a*>(base + at.d);
-      const f32x4a d1 = *reinterpret_cast<const f32x4a*>(base + at.d + 16);
+  for (int c = 0; c < 4; ++c) {
+    const u32x4a v = *reinterpret_cast<const u32x4a*>(base + (SRC == kPacked ? 64 * c * at.nt : 64 * c) + at.q);
+    y.q[c] = i32x4{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+  }
+  if constexpr (FMT == RV_QF_Q8_0) {
+    const f32x4a d0 = *reinterpret_cast<const f32x4a*>(base + at.d);
+    const f32x4a d1 = *reinterpret_cast<const f32x4a*>(base + at.d + 16);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) y.d[c] = d0[c], y.d[4 + c] = d1[c];
-    } else {
-      if constexpr (FMT != RV_QF_Q6_K) y.bs = *reinterpret_cast<const f16x4a*>(base + at.bs);
-      y.d[0] = *reinterpret_cast<const float*>(base + at.d);
-    }
-  } else if constexpr (kQ80) {
-    const rv_block_q8_0* r = reinterpret_cast<const rv_block_q8_0*>(at.base);
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const rv_block_q8_0* b = r + min(8 * step + c, nb - 1);
-      const u32x2a v = *reinterpret_cast<const u32x2a*>(b->qs + 8 * kq);
-      y.q[c >> 1][2 * (c & 1)] = (int)v[0];
-      y.q[c >> 1][2 * (c & 1) + 1] = (int)v[1];
-      y.d[c] = b->d;
-    }
+    for (int c = 0; c < 4; ++c) y.d[c] = d0[c], y.d[4 + c] = d1[c];
   } else {
-    const rv_block_q8_k* b = reinterpret_cast<const rv_block_q8_k*>(at.base);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const u32x4a v = *reinterpret_cast<const u32x4a*>(b->qs + 64 * c + 16 * kq);
-      y.q[c] = i32x4{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
-    }
-    y.d[0] = b->d;
+    if constexpr (FMT != RV_QF_Q6_K && SRC == kPacked) y.bs = *reinterpret_cast<const f16x4a*>(base + at.bs);
+    y.d[0] = *reinterpret_cast<const float*>(base + at.d);
   }
 }
 
+// Public blocks (a row's after one another): loaded 256 contiguous bytes of a
+// row at a time and turned around through the wave's own LDS, written a block
+// ahead of its use and loaded two ahead. In operand order straight from the
+// blocks, a row per lane, each load takes 64 cycles or more of the CU's address
+// unit, for every 16 weight rows again: 4096 x 2048 weights by 512 activations
+// Q4_K 32.8 -> 30.9 us a call, Q8_0 135 -> 40; 8192 x 8192 by 1024 611 -> 390,
+// 1908 -> 491. What binds Q4_K and Q6_K then is the LDS, 16 16-byte accesses a
+// block and wave, so that two row groups share each block (launch_batched).
+constexpr int kTurnRow = 272;  // bytes per row of 256 (16-byte reads of 16 rows and writes of a row: all banks)
+constexpr int kTurnD = 12;     // floats per row of the Q8_0 scales (16-byte reads of 16 rows: all banks)
+constexpr int kTurnScales = 16 * kTurnRow;
+constexpr int kTurnBytes = kTurnScales + 2 * 16 * kTurnD * (int)sizeof(float);  // scales of two groups
+template <int FMT>
+struct TurnedActs {
+  static constexpr bool kQ80 = FMT == RV_QF_Q8_0;
+  const char* base;  // the tile's first row (K: the block last loaded of it): wave-uniform
+  uint32_t off[4];   // the lane's 16 bytes of rows 4 i + lane / 16
+  uint32_t doff[kQ80 ? 2 : 1];
+  int lane, nb;
+  char* lds;
+  u32x4a raw[4];
+  float rd[kQ80 ? 2 : 1], dk;
+
+  __device__ __forceinline__ TurnedActs(const BatchedArgs& a, int tile, int lane_, char* lds_) : lane(lane_), lds(lds_) {
+    nb = a.in_dim / (kQ80 ? 32 : 256);
+    const uint32_t row = (uint32_t)nb * (kQ80 ? sizeof(rv_block_q8_0) : sizeof(rv_block_q8_k));
+    const int nt = min(16, a.n_acts - 16 * tile);
+    base = reinterpret_cast<const char*>(kQ80 ? a.acts_0 : a.acts_k) + (size_t)tile * 16 * row;
+    // Rows past the tile repeat its last. K: chunk lane % 16 of the block. Q8_0:
+    // half lane % 2 of block lane / 2 % 8 of the group (its offset by load).
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      off[i] = row * min(4 * i + (lane >> 4), nt - 1) + 4 + 16 * (kQ80 ? lane & 1 : lane & 15);
+    if constexpr (kQ80) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) doff[i] = row * min(8 * i + (lane >> 3), nt - 1);
+    } else {
+      doff[0] = row * min(lane & 15, nt - 1);
+    }
+    load(0);
+    if constexpr (kQ80) {
+      put(0, raw, rd);
+      load(1);
+    } else {  // the first two in flight together
+      u32x4a first[4];
+      const float fd[1] = {rd[0]};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) first[i] = raw[i];
+      if (nb > 1) base += sizeof(rv_block_q8_k);
+      load(1);
+      put(0, first, fd);
+    }
+  }
+  // Block b (K: the one at base) of the tile's rows; Q8_0: blocks 8 b .. + 7,
+  // those past the row its last.
+  __device__ __forceinline__ void load(int b) {
+    uint32_t at = 0;
+    if constexpr (kQ80) at = (uint32_t)min(8 * b + ((lane >> 1) & 7), nb - 1) * sizeof(rv_block_q8_0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) raw[i] = *reinterpret_cast<const u32x4a*>(base + (off[i] + at));
+    if constexpr (kQ80) {
+      const uint32_t dat = (uint32_t)min(8 * b + (lane & 7), nb - 1) * sizeof(rv_block_q8_0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) rd[i] = *reinterpret_cast<const float*>(base + (doff[i] + dat));
+    } else {
+      rd[0] = *reinterpret_cast<const float*>(base + doff[0]);
+    }
+  }
+  __device__ __forceinline__ float* dd(int k) const {
+    return reinterpret_cast<float*>(lds + kTurnScales) + 16 * kTurnD * (k & 1);
+  }
+  __device__ __forceinline__ void put(int k, const u32x4a (&w)[4], const float (&wd)[kQ80 ? 2 : 1]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 4 * i + (lane >> 4);
+      if constexpr (kQ80) {  // as build0 lays the weights
+        const int c = (lane >> 1) & 7, at = 4 * (c >> 1) + 2 * (lane & 1);
+        *reinterpret_cast<i32x2*>(lds + kTurnRow * r + 16 * at + 8 * (c & 1)) = i32x2{(int)w[i][0], (int)w[i][1]};
+        *reinterpret_cast<i32x2*>(lds + kTurnRow * r + 16 * at + 16 + 8 * (c & 1)) = i32x2{(int)w[i][2], (int)w[i][3]};
+      } else {
+        *reinterpret_cast<i32x4*>(lds + kTurnRow * r + 16 * (lane & 15)) =
+            i32x4{(int)w[i][0], (int)w[i][1], (int)w[i][2], (int)w[i][3]};
+      }
+    }
+    if constexpr (kQ80) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) dd(k)[kTurnD * (8 * i + (lane >> 3)) + (lane & 7)] = wd[i];
+    } else {
+      dk = wd[0];
+    }
+  }
+  // Block b of n into y; b % 2 == k % 2.
+  __device__ __forceinline__ void next(Act<FMT>& y, int k, int b, int n) {
+    const int col = lane & 15, kq = lane >> 4;
+    wave_lds_order();
+#pragma unroll
+    for (int c = 0; c < 4; ++c) y.q[c] = *reinterpret_cast<const i32x4*>(lds + kTurnRow * col + 64 * c + 16 * kq);
+    if constexpr (!kQ80) y.d[0] = dk;
+    wave_lds_order();  // read before the next block goes over it
+    put(k + 1, raw, rd);
+    if (!kQ80 && b + 2 < n) base += sizeof(rv_block_q8_k);
+    load(b + 2);
+  }
+  // Q8_0: the four scales c .. + 3 of the group last taken (which was k).
+  __device__ __forceinline__ f32x4 scales(int k, int c) const {
+    return *reinterpret_cast<const f32x4*>(dd(k) + kTurnD * (lane & 15) + c);
+  }
+};
+
+struct NoTurn {
+  __device__ __forceinline__ NoTurn(const BatchedArgs&, int, int, char*) {}
+};
+template <int FMT, int SRC>
+using Turned = std::conditional_t<SRC == kTurned, TurnedActs<FMT>, NoTurn>;
+
 // The sums of the lane's 16 values of each chunk (carried by the packed
-// layout, formed here from blocks in the public one).
-template <int FMT, bool PACKED>
+// layout, formed here from public blocks).
+template <int FMT, int SRC>
 __device__ __forceinline__ f16x4 act_sums(const Act<FMT>& y) {
-  if constexpr (PACKED) return y.bs;
+  if constexpr (SRC == kPacked) return y.bs;
   f16x4 r;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
@@ -358,72 +458,85 @@ __device__ __forceinline__ void store4(const BatchedArgs& a, const BatchedSeg& s
   }
 }
 
-__device__ __forceinline__ size_t row_at(const BatchedSeg& sg, int i) {
-  return (size_t)(sg.row_lo + min(i, sg.n_rows - 1)) * sg.row_bytes;
-}
-
 // ---- the products ----------------------------------------------------------------
 
-// A k-quant segment's rows 16 rg .. against activation tile kW ag + wave of
-// each wave.
-template <int FMT, bool PACKED>
-__device__ __forceinline__ void kq_body(const BatchedArgs& a, const BatchedSeg& sg, int rg, int ag, Planes& pl) {
+// A k-quant segment's rows 16 RG rg .. against activation tile kW ag + wave of
+// each wave. RG row groups share each block's operands; the planes' KC slots
+// then hold KC / RG blocks of each.
+template <int FMT, int SRC, int RG>
+__device__ __forceinline__ void kq_body(const BatchedArgs& a, const BatchedSeg& sg, int rg, int ag, Planes& pl,
+                                        char* turn) {
 #pragma clang fp contract(off)
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 15, kq = lane >> 4;
   const int nb = a.in_dim / 256, n_tiles = (a.n_acts + 15) / 16, tile = ag * kW + wave;
   // Unpacking: piece tid % 8 (eight lanes read a block's 128 quant bytes) of
-  // row (tid / 8) % 16 and block tid / 128 of the chunk. The rows are taken in
+  // row (tid / 8) % 16 and slot tid / 128 of the planes: row group slot % RG
+  // and block slot / RG of the chunk. The rows are taken in
   // the order that gives neighbouring groups of eight lanes the two halves of
   // the banks: Q6_K's pieces fill chunks 0-3 and 8-11 of a row (swizzled: the
   // others of row ^ 4), the others' 0, 1, 4, 5, .. (of row ^ 2). Rows past the
   // range re-read its last (their outputs are not stored), blocks past the
   // row its last.
-  const int bp = tid & 7, i8 = (tid >> 3) & 15, bk = wave >> 1;
+  constexpr int KB = KC / RG;
+  const int bp = tid & 7, i8 = (tid >> 3) & 15, slot = wave >> 1, bk = slot / RG;
   const int br = FMT == RV_QF_Q6_K ? ((i8 & 1) << 2) | ((i8 & 6) >> 1) | (i8 & 8)
                                    : ((i8 & 1) << 1) | ((i8 & 2) >> 1) | (i8 & 12);
-  const uint8_t* wrow = sg.w + (size_t)(sg.row_lo + min(kR * rg + br, sg.n_rows - 1)) * sg.row_bytes;
+  const uint8_t* wrow = sg.w + (size_t)(sg.row_lo + min(kR * (RG * rg + slot % RG) + br, sg.n_rows - 1)) * sg.row_bytes;
   Raw<FMT> raw;
   load_raw<FMT>(raw, wrow, nb, bk, bp);
-  ActAt at = act_at<FMT, PACKED>(a, min(tile, n_tiles - 1), col, kq);
-  Act<FMT> act[2];
-  load_act<FMT, PACKED>(act[0], at, nb, 0, kq);
-  f32x4 sumf{};
-  for (int b0 = 0; b0 < nb; b0 += KC) {
+  Turned<FMT, SRC> turned(a, min(tile, n_tiles - 1), lane, turn + wave * kTurnBytes);
+  ActAt at;
+  Act<FMT> act[SRC == kTurned ? 1 : 2];
+  if constexpr (SRC != kTurned) {
+    at = act_at<FMT, SRC>(a, min(tile, n_tiles - 1), col, kq);
+    load_act<FMT, SRC>(act[0], at);
+  }
+  f32x4 sumf[RG]{};
+  for (int b0 = 0; b0 < nb; b0 += KB) {
     if (b0) __syncthreads();  // every wave is done with the previous chunk's planes
-    build<FMT>(raw, pl, br, bk, bp);
-    load_raw<FMT>(raw, wrow, nb, b0 + KC + bk, bp);
+    build<FMT>(raw, pl, br, slot, bp);
+    load_raw<FMT>(raw, wrow, nb, b0 + KB + bk, bp);
     __syncthreads();
     if (tile >= n_tiles) continue;  // wave-uniform: a wave without activations only unpacks
+    f16x4 bs;
 #pragma unroll
-    for (int k = 0; k < KC; ++k) {
-      if (b0 + k >= nb) break;
-      if (b0 + k + 1 < nb) at.base += at.step;  // the last block is loaded again, unused
-      load_act<FMT, PACKED>(act[(k + 1) & 1], at, nb, 0, kq);
-      const Act<FMT>& y = act[k & 1];
+    for (int p = 0; p < KC; ++p) {  // the planes' slots
+      const int k = p / RG, g = p % RG;
+      if (g == 0 && b0 + k >= nb) break;
+      if (g == 0) {
+        if constexpr (SRC == kTurned) {
+          turned.next(act[0], k, b0 + k, nb);
+        } else {
+          if (b0 + k + 1 < nb) at.base += at.step;  // the last block is loaded again, unused
+          load_act<FMT, SRC>(act[(k + 1) & 1], at);
+        }
+      }
+      const Act<FMT>& y = act[SRC == kTurned ? 0 : k & 1];
       i32x4 hi{}, lo{};
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const i32x4 wh = *reinterpret_cast<const i32x4*>(&pl.p[k][0][chunk_at(col, 4 * c + kq)]);
-        const i32x4 wl = *reinterpret_cast<const i32x4*>(&pl.p[k][1][chunk_at(col, 4 * c + kq)]);
+        const i32x4 wh = *reinterpret_cast<const i32x4*>(&pl.p[p][0][chunk_at(col, 4 * c + kq)]);
+        const i32x4 wl = *reinterpret_cast<const i32x4*>(&pl.p[p][1][chunk_at(col, 4 * c + kq)]);
         hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(wh, y.q[c], hi, 0, 0, 0);
         lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(wl, y.q[c], lo, 0, 0, 0);
       }
-      const f32x4 dw = *reinterpret_cast<const f32x4*>(&pl.d[k][0][4 * kq]);
+      const f32x4 dw = *reinterpret_cast<const f32x4*>(&pl.d[p][0][4 * kq]);
       const float da = y.d[0];
       if constexpr (FMT == RV_QF_Q6_K) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int sumi = 64 * hi[r] + lo[r];
-          sumf[r] += dw[r] * da * (float)sumi;
+          sumf[g][r] += dw[r] * da * (float)sumi;
         }
       } else {
-        const f32x4 dm = *reinterpret_cast<const f32x4*>(&pl.d[k][1][4 * kq]);
-        const f16x4 m4 = *reinterpret_cast<const f16x4*>(&pl.mins[k][col][4 * (kq >> 1)]);
-        const f16x4 bs = act_sums<FMT, PACKED>(y);
+        const f32x4 dm = *reinterpret_cast<const f32x4*>(&pl.d[p][1][4 * kq]);
+        const f16x4 m4 = *reinterpret_cast<const f16x4*>(&pl.mins[p][col][4 * (kq >> 1)]);
+        if (g == 0) bs = act_sums<FMT, SRC>(y);
         const f32x4 mins = __builtin_amdgcn_mfma_f32_16x16x16f16(m4, bs, f32x4{}, 0, 0, 0);
         int extra = 0;
         if constexpr (FMT == RV_QF_Q5_K) {
+          static_assert(RG == 1, "Q5_K takes one row group");
           const f16x4 one = {(_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f};
           extra = 1152 * (int)__builtin_amdgcn_mfma_f32_16x16x16f16(one, bs, f32x4{}, 0, 0, 0)[0];
         }
@@ -431,17 +544,20 @@ __device__ __forceinline__ void kq_body(const BatchedArgs& a, const BatchedSeg& 
         for (int r = 0; r < 4; ++r) {
           const int sumi = 8 * hi[r] + lo[r] + extra;
           const float d = dw[r] * da, dmin = dm[r] * da;
-          sumf[r] += d * (float)sumi - dmin * mins[r];
+          sumf[g][r] += d * (float)sumi - dmin * mins[r];
         }
       }
+      if constexpr (RG == 2) __builtin_amdgcn_sched_barrier(0);
     }
   }
-  store4(a, sg, kR * rg + 4 * kq, 16 * tile + col, sumf);
+  store4(a, sg, kR * RG * rg + 4 * kq, 16 * tile + col, sumf[0]);
+  if constexpr (RG == 2) store4(a, sg, kR * (RG * rg + 1) + 4 * kq, 16 * tile + col, sumf[1]);
 }
 
 // A Q8_0 segment's 16 rows 16 rg .. against one activation tile per wave.
-template <bool PACKED>
-__device__ __forceinline__ void q80_body(const BatchedArgs& a, const BatchedSeg& sg, int rg, int ag, Planes0& pl) {
+template <int SRC>
+__device__ __forceinline__ void q80_body(const BatchedArgs& a, const BatchedSeg& sg, int rg, int ag, Planes0& pl,
+                                         char* turn) {
 #pragma clang fp contract(off)
   constexpr int FMT = RV_QF_Q8_0, NI = kR * KC * 32 / (64 * kW);
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -456,9 +572,13 @@ __device__ __forceinline__ void q80_body(const BatchedArgs& a, const BatchedSeg&
   Raw<FMT> raw[NI];
 #pragma unroll
   for (int u = 0; u < NI; ++u) load_raw<FMT>(raw[u], wrow[u], nb, bk, bp);
-  ActAt at = act_at<FMT, PACKED>(a, min(tile, n_tiles - 1), col, kq);
-  Act<FMT> act[2];
-  load_act<FMT, PACKED>(act[0], at, nb, 0, kq);
+  Turned<FMT, SRC> turned(a, min(tile, n_tiles - 1), lane, turn + wave * kTurnBytes);
+  ActAt at;
+  Act<FMT> act[SRC == kTurned ? 1 : 2];
+  if constexpr (SRC != kTurned) {
+    at = act_at<FMT, SRC>(a, min(tile, n_tiles - 1), col, kq);
+    load_act<FMT, SRC>(act[0], at);
+  }
   f32x4 sumf{};
   for (int s0 = 0; s0 < steps; s0 += KC) {
     if (s0) __syncthreads();
@@ -472,20 +592,30 @@ __device__ __forceinline__ void q80_body(const BatchedArgs& a, const BatchedSeg&
     for (int k = 0; k < KC; ++k) {
       const int s = s0 + k;
       if (s >= steps) break;
-      if (s + 1 < steps) at.base += at.step;
-      load_act<FMT, PACKED>(act[(k + 1) & 1], at, nb, PACKED ? 0 : min(s + 1, steps - 1), kq);
-      const Act<FMT>& y = act[k & 1];
+      if constexpr (SRC == kTurned) {
+        turned.next(act[0], k, s, steps);
+      } else {
+        if (s + 1 < steps) at.base += at.step;
+        load_act<FMT, SRC>(act[(k + 1) & 1], at);
+      }
+      const Act<FMT>& y = act[SRC == kTurned ? 0 : k & 1];
       const int nblk = min(8, nb - 8 * s);
+      f32x4 dy;
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
+        if constexpr (SRC == kTurned) {
+          if (c % 4 == 0) dy = turned.scales(k, c);
+        } else {
+          dy[c % 4] = y.d[c];
+        }
         const i32x2 w2 = *reinterpret_cast<const i32x2*>(&pl.p[k][chunk_at(col, 4 * (c >> 1) + kq) + 8 * (c & 1)]);
         const i32x2 y2 = {y.q[c >> 1][2 * (c & 1)], y.q[c >> 1][2 * (c & 1) + 1]};
         const i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, w2), __builtin_bit_cast(long, y2),
                                                                 i32x4{}, 0, 0, 0);
         const f32x4 dw = *reinterpret_cast<const f32x4*>(&pl.d[k][c][4 * kq]);
-        if (PACKED || c < nblk) {
+        if (SRC == kPacked || c < nblk) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) sumf[r] += (float)acc[r] * (dw[r] * y.d[c]);
+          for (int r = 0; r < 4; ++r) sumf[r] += (float)acc[r] * (dw[r] * dy[c % 4]);
         }
       }
     }
@@ -493,9 +623,11 @@ __device__ __forceinline__ void q80_body(const BatchedArgs& a, const BatchedSeg&
   store4(a, sg, kR * rg + 4 * kq, 16 * tile + col, sumf);
 }
 
-template <bool PACKED>
+template <int SRC, int RG>
 __global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(4))) void batched_kernel(BatchedArgs a) {
-  __shared__ __attribute__((aligned(16))) char lds[sizeof(Planes) > sizeof(Planes0) ? sizeof(Planes) : sizeof(Planes0)];
+  constexpr int kPlaneBytes = sizeof(Planes) > sizeof(Planes0) ? sizeof(Planes) : sizeof(Planes0);
+  static_assert(kPlaneBytes % 16 == 0 && kTurnBytes % 16 == 0, "16-byte LDS accesses");
+  __shared__ __attribute__((aligned(16))) char lds[kPlaneBytes + (SRC == kTurned ? kW * kTurnBytes : 0)];
   int b = (int)blockIdx.x, si = 0;
   while (si + 1 < a.n_seg && b >= a.seg[si].blocks) b -= a.seg[si++].blocks;
   const BatchedSeg& sg = a.seg[si];
@@ -506,11 +638,17 @@ __global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(4))) vo
   const int rg = 8 * q8 + rem % 8, ag = rem / 8;
   if (rg >= sg.n_rg) return;  // uniform: the last eight row groups may be partial
   auto& pl = *reinterpret_cast<Planes*>(lds);
+  char* const turn = lds + kPlaneBytes;  // each wave's activations (turned)
+  // (The launch takes Q8_0 and Q5_K to the instantiations that have them.)
   switch (sg.fmt) {
-    case RV_QF_Q8_0: return q80_body<PACKED>(a, sg, rg, ag, *reinterpret_cast<Planes0*>(lds));
-    case RV_QF_Q4_K: return kq_body<RV_QF_Q4_K, PACKED>(a, sg, rg, ag, pl);
-    case RV_QF_Q5_K: return kq_body<RV_QF_Q5_K, PACKED>(a, sg, rg, ag, pl);
-    default: return kq_body<RV_QF_Q6_K, PACKED>(a, sg, rg, ag, pl);
+    case RV_QF_Q8_0:
+      if constexpr (RG == 1 && SRC != kDirect) q80_body<SRC>(a, sg, rg, ag, *reinterpret_cast<Planes0*>(lds), turn);
+      return;
+    case RV_QF_Q4_K: return kq_body<RV_QF_Q4_K, SRC, RG>(a, sg, rg, ag, pl, turn);
+    case RV_QF_Q5_K:
+      if constexpr (RG == 1) kq_body<RV_QF_Q5_K, SRC, RG>(a, sg, rg, ag, pl, turn);
+      return;
+    default: return kq_body<RV_QF_Q6_K, SRC, RG>(a, sg, rg, ag, pl, turn);
   }
 }
 
@@ -521,17 +659,40 @@ HipStatus launch_batched(BatchedArgs a, bool packed, hipStream_t s) {
   if (a.n_acts == 0 || a.in_dim == 0) return st;
   unsigned grid = 0;
   a.n_ag = (a.n_acts + 16 * kW - 1) / (16 * kW);
+  // Public blocks (one segment). With up to two working waves a CU the turn's
+  // latency shows, and k-quants load in operand order. Turned vs not, us per
+  // call: Q4_K 4096 x 2048 weights, 1 activation 7.7 vs 7.2, 32 (512 waves) 8.3
+  // vs 8.0, 128 11.3 vs 12.0; 8192 x 8192, 16 (512) 23.6 vs 23.0, 32 27.6 vs 30.8.
+  // Q8_0's scattered 8-byte loads lose there too (4096 x 2048, 1 12.2 vs 13.1).
+  const BatchedSeg& s0 = a.seg[0];
+  const long waves = (long)((s0.n_rows + kR - 1) / kR) * ((a.n_acts + 15) / 16);
+  const bool direct = !packed && s0.fmt != RV_QF_Q8_0 && waves <= 512;
+  // Otherwise Q4_K and Q6_K take two row groups a workgroup once one would put
+  // two workgroups on a CU, with at least half of the waves at work. One vs
+  // two: Q4_K 4096 x 2048, 128 activations (256 workgroups) 11.3 vs 14.3, 256
+  // 17.0 vs 14.8, 512 30.9 vs 23.2; 8192 x 8192, 32 27.6 vs 30.0, 64 34.2 either
+  // way, 1024 390 vs 283; Q6_K 410 vs 297. (Q5_K's registers do not allow it;
+  // Q8_0 is bound by its float work.)
+  const long pairs = (long)((s0.n_rows + 2 * kR - 1) / (2 * kR)) * a.n_ag;
+  const bool two = !packed && !direct && (s0.fmt == RV_QF_Q4_K || s0.fmt == RV_QF_Q6_K) && pairs > 128 && a.n_acts >= 64;
+  const int rows = two ? 2 * kR : kR;
   for (int i = 0; i < a.n_seg; ++i) {
     BatchedSeg& g = a.seg[i];
-    g.n_rg = (g.n_rows + kR - 1) / kR;
+    g.n_rg = (g.n_rows + rows - 1) / rows;
     g.blocks = (g.n_rg + 7) / 8 * 8 * a.n_ag;
     grid += (unsigned)g.blocks;
   }
   if (grid == 0) return st;
+#define RV_BATCHED(SRC, RG) hipLaunchKernelGGL((batched_kernel<SRC, RG>), dim3(grid), dim3(64 * kW), 0, s, a)
   if (packed)
-    hipLaunchKernelGGL(batched_kernel<true>, dim3(grid), dim3(64 * kW), 0, s, a);
+    RV_BATCHED(kPacked, 1);
+  else if (direct)
+    RV_BATCHED(kDirect, 1);
+  else if (two)
+    RV_BATCHED(kTurned, 2);
   else
-    hipLaunchKernelGGL(batched_kernel<false>, dim3(grid), dim3(64 * kW), 0, s, a);
+    RV_BATCHED(kTurned, 1);
+#undef RV_BATCHED
   st.e = hipGetLastError();
   if (st.e != hipSuccess) st.what = "batched gemv launch";
   return st;

@@ -206,3 +206,39 @@ def test_rows_projections_at_tile_edges(q_fmt, v_fmt, n, blocks):
     for got, fmt, w, m, acts in ((q, q_fmt, wq, q_dim, ak), (k, Q.RV_QF_Q8_0, wk, kv_dim, a0), (v, v_fmt, wv, kv_dim, ak)):
         want = oracle.gemv(fmt, w, hidden, m, acts, n_acts=n, rows=(0, m)).reshape(m, n).T
         assert got.cpu().numpy().tobytes() == np.ascontiguousarray(want).tobytes(), f"fmt {fmt}"
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("out_dim,in_dim,n_acts", [(520, 256, 240), (520, 256, 241), (2050, 1280, 80), (4096, 256, 63),
+                                                   (4097, 256, 64), (4113, 768, 65), (4128, 512, 129)])
+def test_batched_gemv_around_the_lines_of_its_forms(fmt, out_dim, in_dim, n_acts):
+    """Public blocks loaded in operand order (up to 512 row group x activation
+    tile pairs), turned around in LDS, and with two row groups a workgroup
+    (more than 128 pairs of groups, 64 activations): both sides of each line,
+    partial pairs, 1 to 5 blocks (chunks of four and of two), activations of
+    -128 throughout (sums of -2048) beside random ones. Three windows of rows."""
+    torch = torch_cuda()
+    say(f"case batched lines fmt={fmt} {out_dim}x{in_dim} x {n_acts}")
+    rng = np.random.default_rng(out_dim + in_dim + n_acts + fmt)
+    w = random_weight_rows(fmt, out_dim, in_dim, rng)
+    acts = quantize_rows(fmt, rng.standard_normal((n_acts, in_dim)).astype(F32))
+    acts["qs"][-1] = -128
+    if "bsums" in acts.dtype.names:
+        acts["bsums"][-1] = -2048
+    got = run_batched(torch, fmt, w, in_dim, out_dim, acts, n_acts, (0, out_dim)).reshape(out_dim, n_acts)
+    assert not np.isnan(got).any()
+    for lo in (0, out_dim // 2, out_dim - 33):
+        want = oracle.gemv(fmt, w, in_dim, out_dim, acts, n_acts=n_acts, rows=(lo, lo + 33)).reshape(33, n_acts)
+        assert got[lo:lo + 33].tobytes() == want.tobytes(), f"rows {lo}"
+
+
+@pytest.mark.parametrize("in_dim,n_acts", [(32, 1), (256, 16), (288, 17), (1056, 130), (1312, 33)])
+def test_batched_q8_0_turned_at_partial_groups(in_dim, n_acts):
+    """Q8_0's groups of eight blocks: 1, 8, 9, 33 and 41 blocks a row."""
+    torch = torch_cuda()
+    say(f"case batched Q8_0 {in_dim} x {n_acts}")
+    rng = np.random.default_rng(in_dim + n_acts)
+    fmt = oracle.RV_QF_Q8_0
+    w = random_weight_rows(fmt, 35, in_dim, rng)
+    acts = quantize_rows(fmt, rng.standard_normal((n_acts, in_dim)).astype(F32))
+    check(torch, fmt, w, in_dim, 35, acts, n_acts)
