@@ -746,6 +746,11 @@ HipStatus launch_quantize_rows(const float* x, size_t n_rows, size_t n, const fl
                                void* packed_0, hipStream_t s) {
   HipStatus st;
   if (n_rows == 0 || n == 0) return st;
+  if (norm_w && !packed_0) {  // the normed form writes both
+    st.e = hipErrorInvalidValue;
+    st.what = "quantize rows: the norm without the Q8_0 rows";
+    return st;
+  }
   char *pk = (char*)packed_k, *p0 = (char*)packed_0;
   const unsigned nb = (unsigned)(n / 256);
   if (norm_w)
