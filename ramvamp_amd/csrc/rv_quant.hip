@@ -412,27 +412,6 @@ __global__ __launch_bounds__(64 * kRowsPerWG) void gemv_rows_kernel(const uint8_
   if (lane == 0) out[i] = v;
 }
 
-// 1 / sqrt(mean(x^2) + eps) of n values, as norm.rs:18-26 computes it: the
-// squares summed in f64 (here per thread, then over lanes and waves in a
-// fixed order, so every thread of the workgroup gets the same value), sqrt
-// and reciprocal in f64, rounded once to f32. `red` holds NT / 64 doubles.
-template <int NT>
-__device__ __forceinline__ float block_inv_rms(const float* __restrict__ x, int n, float eps, double* red) {
-  double ss = 0.0;
-  for (int i = threadIdx.x; i < n; i += NT) {
-    const double v = (double)x[i];
-    ss += v * v;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  double tot = 0.0;
-#pragma unroll
-  for (int w = 0; w < NT / 64; ++w) tot += red[w];
-  return (float)(1.0 / sqrt(tot / (double)n + (double)eps));
-}
-
 // Sum over the wave in the order of a shuffle tree over lanes 32, 16, .., 1
 // apart, by swaps and DPP (after the first three steps the values repeat every
 // eight lanes, so a rotation by 4 reaches the lane 4 apart).
@@ -554,10 +533,25 @@ __global__ __launch_bounds__(64 * kFusedWaves) void fused_proj_kernel(FusedProjA
   }
 }
 
+// norm.rs:18-58: 1 / sqrt(mean(x^2) + eps) with the squares summed in f64 (here
+// per thread, then over lanes and waves in a fixed order, so every thread gets
+// the same value), sqrt and reciprocal in f64, rounded once to f32.
 __global__ __launch_bounds__(1024) void rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                        float eps, int n, float* __restrict__ out) {
   __shared__ double red[16];
-  const float inv = block_inv_rms<1024>(x, n, eps, red);
+  double ss = 0.0;
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    const double v = (double)x[i];
+    ss += v * v;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  double tot = 0.0;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) tot += red[v];
+  const float inv = (float)(1.0 / sqrt(tot / (double)n + (double)eps));
   for (int j = threadIdx.x; j < n; j += 1024) {
 #pragma clang fp contract(off)
     out[j] = x[j] * inv * w[j];
@@ -591,7 +585,9 @@ __global__ __launch_bounds__(64 * W) void quantize_rows_kernel(const float* __re
   float inv = 1.f;
   if constexpr (NORM) {
     __shared__ double red[4];
-    if (wave < 4) {  // 256 threads, in the order of rmsnorm_kernel's 256-thread form
+    // The squares in f64: thread t < 256 takes t, t + 256, .., then each wave's
+    // sum, then the four waves' in order.
+    if (wave < 4) {
       double ss = 0.0;
       for (int i = threadIdx.x; i < n; i += 256) {
         const double v = (double)xr[i];

@@ -15,7 +15,6 @@ namespace rv {
 // = nb0 * 32 values, at most kFusedMaxKBlocks * 256.
 constexpr int kFusedWaves = 8;
 constexpr int kFusedMaxKBlocks = 32;
-constexpr int kFusedMax0Blocks = kFusedMaxKBlocks * 8;
 // With norm_w set, x is first RMS-normalized (norm.rs:18-58: f64 mean of
 // squares, x * inv * w in f32) in registers, and the normalized row is what
 // gets quantized. With a segment's `add` set, its rows store add[i] + dot
