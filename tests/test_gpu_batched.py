@@ -242,3 +242,21 @@ def test_batched_q8_0_turned_at_partial_groups(in_dim, n_acts):
     w = random_weight_rows(fmt, 35, in_dim, rng)
     acts = quantize_rows(fmt, rng.standard_normal((n_acts, in_dim)).astype(F32))
     check(torch, fmt, w, in_dim, 35, acts, n_acts)
+
+
+@pytest.mark.parametrize("fmt", FORMATS[:3])
+@pytest.mark.parametrize("n,width,blocks", [(1, 17, 1), (17, 42, 5), (130, 33, 9)])
+def test_out_projection_rows_at_ragged_widths(fmt, n, width, blocks):
+    """The residual add of the output projection's rows where the last four
+    columns of a lane are partial: widths not divisible by 4 or 16."""
+    torch = torch_cuda()
+    say(f"case out projection rows fmt={fmt} n={n} width={width}")
+    rng = np.random.default_rng(0x0D + n + width + fmt)
+    q_dim = 256 * blocks
+    w = random_weight_rows(fmt, width, q_dim, rng)
+    x = rng.standard_normal((n, q_dim)).astype(F32)
+    res = rng.standard_normal((n, width)).astype(F32)
+    dev = torch.from_numpy(res.copy()).cuda()
+    P.attn_out_proj_rows(torch.from_numpy(x).cuda(), fmt, dev_u8(torch, w), dev)
+    o = oracle.gemv(fmt, w, q_dim, width, quantize_rows(fmt, x), n_acts=n, rows=(0, width)).reshape(width, n).T
+    assert dev.cpu().numpy().tobytes() == np.ascontiguousarray(res + o).tobytes()

@@ -240,3 +240,43 @@ def test_attn_block_prefill_matches_the_oracle_composition(mode, tol):
         assert err <= tol, f"{mode} chunk {chunk}"
         assert kv.len(1) == start + n and kv.len(0) == n_pos
         start += n
+
+
+@pytest.mark.parametrize("hidden,n_heads,n_kv,n", [(256, 2, 1, 129), (2304, 8, 1, 17), (2304, 4, 2, 1), (4352, 4, 2, 129)])
+def test_attn_block_prefill_projections_at_other_widths(hidden, n_heads, n_kv, n):
+    """Rows of 1, 9 and 17 activation blocks through the normed rows quantizer's
+    8 waves (idle waves, a second and a third round), whole and ragged tiles: the
+    q, k and v rows the call leaves in its scratch, byte for byte, and the
+    residual as above."""
+    torch = torch_cuda()
+    say(f"case prefill block hidden={hidden} heads={n_heads}/{n_kv} rows={n}")
+    Q = oracle
+    rng = np.random.default_rng(0xB11 + hidden + n)
+    hd, start = 128, 21
+    q_dim, kv_dim = n_heads * hd, n_kv * hd
+    lay = Layer(torch, rng, hidden, q_dim, kv_dim, hd, Q.RV_QF_Q5_K, Q.RV_QF_Q6_K, Q.RV_QF_Q4_K)
+    kv, ref = twin(Rng(0xB2), 1, n_kv, hd, start, start + n, "f32")
+    scale = float(np.float32(1.0 / np.sqrt(hd)))
+    res = (1.5 * rng.standard_normal((n, hidden))).astype(np.float32)
+    res[0, :] = 0.0  # a row whose norm is that of eps alone
+    res_dev = torch.from_numpy(res.copy()).cuda()
+    scratch = torch.zeros(B.prefill_scratch_bytes(n, hidden, q_dim, kv_dim), dtype=torch.uint8, device="cuda")
+    B.attn_block_prefill(kv, 0, res_dev, q_dim, lay.dev, EPS, THETA, start, scale, scratch=scratch)
+    torch.cuda.synchronize()
+    normed = [oracle.rmsnorm(r, lay.attn_norm, EPS) for r in res]
+    ak = [oracle.quantize_row_q8_k(x) for x in normed]
+    a0 = [oracle.quantize_row_q8_0(x) for x in normed]
+    q = np.stack([oracle.gemv(lay.q_fmt, lay.wq, hidden, q_dim, a) for a in ak])
+    k = np.stack([oracle.gemv(Q.RV_QF_Q8_0, lay.wk, hidden, kv_dim, a) for a in a0])
+    v = np.stack([oracle.gemv(lay.v_fmt, lay.wv, hidden, kv_dim, a) for a in ak])
+    held, off = scratch.cpu().numpy(), (n * hidden * 4 + 255) // 256 * 256
+    for name, want in (("q", q), ("k", k), ("v", v)):
+        got = held[off:off + want.nbytes].view(np.float32).reshape(want.shape)
+        bad = np.flatnonzero((got.view(np.uint32) != want.view(np.uint32)).any(1))
+        assert bad.size == 0, f"{name} rows {bad[:8]} of {n}"
+        off += (want.nbytes + 255) // 256 * 256
+    attn = ref.prefill_chunk(0, q, k, v, lay.q_norm, lay.k_norm, EPS, THETA, start, scale)
+    o = np.stack([oracle.gemv(lay.o_fmt, lay.wo, q_dim, hidden, oracle.quantize_row_q8_k(a)) for a in attn])
+    err = np.max(np.abs(res_dev.cpu().numpy().astype(np.float64) - (res + o))) / np.max(np.abs(o))
+    say(f"prefill block hidden={hidden}: residual max|err|/max|o| {err:.2e}")
+    assert err <= 2e-3

@@ -270,3 +270,58 @@ def test_fused_projections_at_ragged_row_counts(hidden, q_dim, kv_dim):
         assert k.cpu().numpy().tobytes() == oracle.gemv(oracle.RV_QF_Q8_0, wk, hidden, kv_dim, acts_0).tobytes()
         want = oracle.gemv(v_fmt, wv, hidden, kv_dim, acts_k).tobytes()
         assert v.cpu().numpy().tobytes() == want and o.cpu().numpy().tobytes() == want
+
+
+def nonfinite_rows(hidden, rng):
+    """Rows with infinities and NaNs in a few blocks, finite values in the others."""
+    x = rng.standard_normal((5, hidden)).astype(F32)
+    x[0, 5], x[0, 133] = np.inf, -np.inf  # the first of equal magnitudes
+    x[1, 40], x[1, 200] = -np.inf, np.nan
+    x[2, 3::7] = np.nan
+    x[3, hidden - 256:] = np.where(np.arange(256) % 32 == 31, F32(0.5), F32(np.nan))
+    x[4, :hidden // 2] = 0.0
+    x[4, hidden // 2 + 9] = np.nan
+    return x
+
+
+def q8_k_blocks(x):
+    """quantize_row_q8_k's blocks, with 0 where a value times the inverse scale
+    is NaN (an integer cast in the reference; undefined in the oracle's C)."""
+    blocks = oracle.quantize_row_q8_k(x)
+    for b, v in zip(blocks, x.reshape(-1, 256)):
+        mag = np.where(np.isnan(v), F32(0), np.abs(v))
+        if mag.max() > 0:
+            with np.errstate(invalid="ignore"):
+                t = F32(-127.0) / v[int(mag.argmax())] * v
+            b["qs"][np.isnan(t)] = 0
+            b["bsums"] = b["qs"].reshape(16, 16).astype(np.int16).sum(1)
+    return blocks
+
+
+def test_quantizers_with_infinities_and_nans():
+    """Both quantizers as calls of their own, in the fused projections and in
+    the rows quantizer: NaN is never the largest, an infinity makes the others 0."""
+    torch = torch_cuda()
+    hidden, dim = 1024, 24
+    rng = np.random.default_rng(0x1F)
+    x = nonfinite_rows(hidden, rng)
+    wq = random_weight_rows(oracle.RV_QF_Q6_K, dim, hidden, rng)
+    wk = random_weight_rows(oracle.RV_QF_Q8_0, dim, hidden, rng)
+    wv = random_weight_rows(oracle.RV_QF_Q4_K, dim, hidden, rng)
+    rows = [torch.empty((len(x), dim), device="cuda") for _ in range(3)]
+    P.attn_in_proj_rows(torch.from_numpy(x).cuda(), oracle.RV_QF_Q6_K, u8(torch, wq), rows[0], u8(torch, wk), rows[1],
+                        oracle.RV_QF_Q4_K, u8(torch, wv), rows[2])
+    for r, row in enumerate(x):
+        say(f"case non-finite row {r}")
+        ak, a0 = q8_k_blocks(row), oracle.quantize_row_q8_0(row)
+        assert gpu_quantize(torch, oracle.RV_QF_Q8_K, row).tobytes() == ak.tobytes()
+        assert gpu_quantize(torch, oracle.RV_QF_Q8_0, row).tobytes() == a0.tobytes()
+        one = [torch.empty(dim, device="cuda") for _ in range(3)]
+        P.attn_in_proj(f32(torch, row), oracle.RV_QF_Q6_K, u8(torch, wq), one[0], u8(torch, wk), one[1],
+                       oracle.RV_QF_Q4_K, u8(torch, wv), one[2])
+        for i, (fmt, w, acts) in enumerate(((oracle.RV_QF_Q6_K, wq, ak), (oracle.RV_QF_Q8_0, wk, a0),
+                                            (oracle.RV_QF_Q4_K, wv, ak))):
+            want = oracle.gemv(fmt, w, hidden, dim, acts)
+            for got in (one[i].cpu().numpy(), rows[i][r].cpu().numpy()):
+                nan = np.isnan(want)
+                assert np.array_equal(np.isnan(got), nan) and got[~nan].tobytes() == want[~nan].tobytes(), (r, i)
