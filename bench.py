@@ -490,7 +490,7 @@ def bench_prefill_projections(torch, rv, iters=20, n_rows=512, n_sets=24):
     ops = 2 * n_rows * (H * (Q + 2 * KV) + Q * H)  # int8 multiply-adds of the exact dots, x2
     return {"us_per_layer": round(per * 1e6, 3), "rows": n_rows, "int8_tops": round(ops / per / 1e12, 2),
             "weight_bytes_per_layer": wbytes, "weight_gbs": round(wbytes / per / 1e9, 1),
-            "launches_per_layer": 7, "distinct_layers": n_sets}
+            "launches_per_layer": 4, "distinct_layers": n_sets}
 
 
 def bench_attn_block_prefill(torch, rv, synth, mode="f16", iters=20):

@@ -91,9 +91,9 @@ int32_t rv_attn_block_decode_dev(rv_kv* kv, size_t layer, float* residual, size_
  * RoPE, append and causal attention (rv_prefill_chunk; flags carries its
  * RV_PREFILL_* mode), and the batched output projection added into each
  * residual row (rv_attn_out_proj_rows). residual_rows[n_rows][hidden] is
- * updated in place; start must equal the layer's length. Launches: the row
- * norm, two quantizers, three batched GEMVs, the prefill chunk's, one
- * quantizer and one batched GEMV. */
+ * updated in place; start must equal the layer's length. Launches: the rows
+ * quantizer (with the norm, both forms), the q, k and v products in one, the
+ * prefill chunk's, the rows quantizer and the output product. */
 size_t rv_attn_block_prefill_scratch_bytes(size_t n_rows, size_t hidden, size_t q_dim, size_t kv_dim);
 int32_t rv_attn_block_prefill(rv_kv* kv, size_t layer, float* residual_rows, size_t n_rows, size_t hidden,
                               size_t q_dim, const rv_attn_block_weights* w, float eps, float theta, size_t start,

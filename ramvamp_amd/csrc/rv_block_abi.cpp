@@ -133,8 +133,9 @@ int32_t rv_attn_block_decode_dev(rv_kv* kv, size_t layer, float* residual, size_
                       scratch_len, flags, err);
 }
 
-// The prefill chunk's scratch: normalized rows, q/k/v rows, attention rows,
-// then the projections' quantized rows.
+// The prefill chunk's scratch: n_rows * hidden floats (unused since the rows
+// quantizer takes the norm; still counted, so that the size and what is refused
+// stay), q/k/v rows, attention rows, then the projections' quantized rows.
 size_t rv_attn_block_prefill_scratch_bytes(size_t n_rows, size_t hidden, size_t q_dim, size_t kv_dim) {
   const size_t proj = std::max(rv::in_proj_rows_scratch_bytes(n_rows, hidden), rv::out_proj_rows_scratch_bytes(n_rows, q_dim));
   return align256(n_rows * hidden * 4) + 2 * align256(n_rows * q_dim * 4) + 2 * align256(n_rows * kv_dim * 4) +
@@ -150,7 +151,7 @@ int32_t rv_attn_block_prefill(rv_kv* kv, size_t layer, float* residual_rows, siz
   if (hidden == 0) return fail(err, RV_PRIM_EMPTY, 0, 0, "rmsnorm");
   const size_t kv_dim = kv->kv_dim, n = n_rows;
   char* p = (char*)scratch;
-  p += align256(n * hidden * 4);  // (held the normed rows; the quantizer norms them now)
+  p += align256(n * hidden * 4);
   float* q = (float*)p;
   p += align256(n * q_dim * 4);
   float* k = (float*)p;

@@ -287,9 +287,11 @@ struct Chunk<_Float16> {
 // One workgroup of W waves per (kv head, split); the `group` (<= 16) query
 // heads of the kv head are the 16 columns of fp32 MFMA tiles
 // (v_mfma_f32_16x16x4_f32: exact fp32 products, fp32 accumulation). Wave w
-// takes the split's 16-position tiles w, w+W, ...; every operand comes
-// straight from global memory into registers, 16 bytes per load, in the
-// layout the MFMA consumes, so nothing is staged through LDS:
+// takes the split's 16-position tiles w, w+W, ...; every operand comes from
+// global memory into registers, 16 bytes per load, no tile staged for the
+// workgroup. V, and with !TURN also q and K, come in the layout the MFMA
+// consumes; with TURN the wave loads q and K in row order and turns them around
+// in its own LDS:
 //   S^T[t][m] = sum_d K[t][d] Q[m][d]: 32 MFMAs; lane (t, k) holds K row t
 //     and lane (m, k) holds q head m at d = E*(k + 4*(s/E)) + s%E for step
 //     s (E = elements per 16-byte chunk), i.e. chunks k, k+4, ... of the row;

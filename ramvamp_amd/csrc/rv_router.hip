@@ -3,14 +3,13 @@
 //
 // Every expert's logit is one serial f32 sum in index order, each product
 // rounded before it is added (dot_f32, forward.rs:1231-1238; contraction off),
-// so the order binds it: a dependent f32 addition takes 9 cycles, 18.4 k for a
-// 2048-wide row.
+// so the order binds it: a dependent f32 addition takes 9 cycles, 18.4 k (7.7
+// us) for a 2048-wide row.
 //
 // At most 128 experts (staged_kernel): two waves per row, lane = expert, take
 // the sums from 64-value chunks of all weight rows that four more waves bring
 // through LDS; each value costs one multiplication (x broadcast from a
-// register by DPP) and one addition, so the wave issues just above the
-// addition's latency. Each row's softmax and top-k then run in one wave with
+// register by DPP) and one addition, the pair 5.4 ns (13 cycles). Each row's softmax and top-k then run in one wave with
 // two experts per lane.
 //
 // Otherwise (router_kernel): each thread streams its own experts' rows with
@@ -378,7 +377,7 @@ __device__ __forceinline__ void choose(StagedLds<R>& s, int r, int lane, int n_e
 // R rows per workgroup: waves 2 r and 2 r + 1 sum row r's experts 0-63 and
 // 64-127, the last kStagers waves bring the weights. Bound by the sums' order:
 // an addition beside the next product takes 5.4 ns, so 11.1 us for 2048 values,
-// of 18.4 us a call for 1 row, 21.8 for 512 and 27.0 for 1024 (31.4, 44.9 and
+// of 18.3 us a call for 1 row, 21.3 for 512 and 26.9 for 1024 (31.4, 47.0 and
 // 58.7 when two waves both staged and summed, each product beside the addition
 // that takes it, one thread took the maximum and the f64 sum, and the top-k
 // went through LDS). Products formed by the stagers, so that the sum waves only
