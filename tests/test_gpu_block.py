@@ -245,7 +245,7 @@ def test_attn_block_prefill_matches_the_oracle_composition(mode, tol):
 @pytest.mark.parametrize("hidden,n_heads,n_kv,n", [(256, 2, 1, 129), (2304, 8, 1, 17), (2304, 4, 2, 1), (4352, 4, 2, 129)])
 def test_attn_block_prefill_projections_at_other_widths(hidden, n_heads, n_kv, n):
     """Rows of 1, 9 and 17 activation blocks through the normed rows quantizer's
-    8 waves (idle waves, a second and a third round), whole and ragged tiles: the
+    8 waves (idle waves, a second and a third pass), whole and ragged tiles: the
     q, k and v rows the call leaves in its scratch, byte for byte, and the
     residual as above."""
     torch = torch_cuda()
